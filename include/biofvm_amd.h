@@ -247,7 +247,8 @@ int bfa_synchronize(bfa_env *env);
 /* Measurement helpers.  bfa_time_kernels runs `reps` diffusion+agent steps
  * with one HIP event pair around every kernel on the handle's stream and
  * returns the mean milliseconds per launch in ms[5] = {x sweep, y sweep,
- * z sweep, agents, whole step}.  bfa_copy_kernel times a plain device copy of
+ * z sweep, agents, whole step}; where x and y are swept by one kernel, ms[0]
+ * holds both and ms[1] an empty event pair.  bfa_copy_kernel times a plain device copy of
  * `bytes` bytes `reps` times (for calibrating HBM byte counters) and returns
  * the mean milliseconds per launch; bfa_copy_kernel_stream does the same with
  * the fastest copy form measured here (one pass, four 16-byte vectors per
@@ -264,7 +265,9 @@ int bfa_copy_kernel_stream(size_t bytes, int reps, double *ms);
  * x-sweep form: rows_x == 0 selects the wave-local x sweep (a row's chunks
  * live in one wavefront), rows_x in {1,2,4,...,64} the LDS-tiled x sweep
  * with that many rows per tile; cols_y / cols_z, the x-columns per y / z
- * sweep block (16, 32 or 64; 0 = automatic).  On error the previous shape is
+ * sweep block (16, 32 or 64; 0 = automatic).  With all six 0 (the default) x
+ * and y of a k-plane are swept by one kernel where that is faster; a shape
+ * set here is one of the separate sweeps.  On error the previous shape is
  * kept.  bfa_get_tiles writes {Lx, Ly, Lz, rows_x, cols_y, cols_z}. */
 int bfa_set_tiles(bfa_env *env, int Lx, int Ly, int Lz, int rows_x, int cols_y, int cols_z);
 int bfa_get_tiles(const bfa_env *env, int *out6);

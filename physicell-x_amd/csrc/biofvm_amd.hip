@@ -20,6 +20,7 @@
 #include "biofvm_amd.h"
 #include "biofvm_aux_kernels.h"
 #include "biofvm_batch_kernels.h"
+#include "biofvm_fused_kernels.h"
 #include "biofvm_kernels.h"
 #include "biofvm_transfer.inc"
 
@@ -43,6 +44,15 @@ constexpr int kXWaveLs[] = {4, 8, 16, 20, 28, 32};
 // Elements of zeroed slack after every device field: the x sweeps load whole
 // row chunks (up to 31 nodes past a row's end) and never store there.
 constexpr size_t kFieldSlack = 64;
+
+// The fused x + y sweep of an environment's default schedule
+// (biofvm_fused_host.inc): fixed by its grid and precision.
+struct FusedPlan {
+    bool on = false;
+    int L = 0, LY = 0, PY = 0, W = 0, threads = 0;  // kernel shape (PlaneArgs)
+    size_t lds = 0;
+    void* sm = nullptr;  // multipliers of the x scans, [ns][12][P]
+};
 
 struct bfa_env {
     int nx = 0, ny = 0, nz = 0, ns = 0;
@@ -123,6 +133,7 @@ struct bfa_env {
     int variant = BFA_LOD_3D_BLOCKING;  // which reference solver's Dirichlet passes
     bool keep_first_dt = false;  // reference caching: coefficients of the first dt kept for later dts
     int slab = 0;  // k-planes per x/y slab pair (0: whole-volume sweeps)
+    FusedPlan xy;
     int split = 1;  // substrate groups swept on parallel streams (1 or 2)
     int runs[3] = {1, 1, 1};  // y / z sweeps: tile sub-runs per XCD (bfa_set_col_runs)
 
@@ -527,6 +538,8 @@ int launch_sweep_win(bfa_env* e, int axis, hipStream_t st, const Win& w) {
                                : launch_sweep<double>(e, axis, st, w);
 }
 
+#include "biofvm_fused_host.inc"
+
 // x and y sweeps in k-slabs of e->slab planes, per substrate, alternating
 // between two side streams so the x sweep of one slab overlaps the y sweep of
 // another; the y sweep of a slab re-reads what its x sweep just wrote while
@@ -540,6 +553,11 @@ int enqueue_xy_slabs(bfa_env* e) {
         for (int k0 = 0; k0 < e->nz; k0 += e->slab, ++q) {
             const int k1 = std::min(e->nz, k0 + e->slab);
             hipStream_t st = e->aux[q & 1];
+            if (fused_active(e)) {
+                int rc = launch_fused_xy(e, st, d, 1, k0, k1 - k0);
+                if (rc) return rc;
+                continue;
+            }
             const Win wx{d, 1, (long long)k0 * e->ny, (long long)(k1 - k0) * e->ny};
             const Win wy{d, 1, (long long)k0 * e->nx, (long long)(k1 - k0) * e->nx};
             int rc = launch_sweep_win(e, 0, st, wx);
@@ -569,10 +587,11 @@ int enqueue_split(bfa_env* e, bool agents) {
         hipStream_t st = e->aux[g];
         HIP_TRY(e, hipStreamWaitEvent(st, e->ev_fork, 0));
         const int d0 = g == 0 ? 0 : h, nd = g == 0 ? h : e->ns - h;
-        for (int a = 0; a < 3; ++a) {
-            int rc = launch_sweep_win(e, a, st, Win{d0, nd, 0, axis_lines(e, a)});
-            if (rc) return rc;
-        }
+        const bool fused = fused_active(e);
+        int rc = fused ? launch_fused_xy(e, st, d0, nd, 0, e->nz) : BFA_OK;
+        for (int a = fused ? 2 : 0; a < 3 && rc == BFA_OK; ++a)
+            rc = launch_sweep_win(e, a, st, Win{d0, nd, 0, axis_lines(e, a)});
+        if (rc) return rc;
         if (agents) {
             int rc = launch_agents_win(e, st, d0, nd);
             if (rc) return rc;
@@ -710,7 +729,7 @@ int run_precompute(bfa_env* e, double dt) {
                            reinterpret_cast<T*>(e->kT), reinterpret_cast<T*>(e->betaT));
         LAUNCH_CHECK(e, "thomas precompute");
     }
-    return BFA_OK;
+    return fused_precompute<T>(e);
 }
 
 int ensure_precompute(bfa_env* e, double dt) {
@@ -762,6 +781,10 @@ int enqueue_diffusion(bfa_env* e) {
         int rc = enqueue_xy_slabs(e);
         if (rc) return rc;
         return launch_sweep_any(e, 2);
+    }
+    if (fused_active(e)) {
+        int rc = launch_fused_xy(e, e->stream, 0, e->ns, 0, e->nz);
+        return rc ? rc : launch_sweep_any(e, 2);
     }
     for (int a = 0; a < 3; ++a) {
         int rc = launch_sweep_any(e, a);
@@ -942,6 +965,7 @@ int bfa_create(bfa_env** out, int nx, int ny, int nz, int ns, double dx, int pre
         (rc = dalloc(e, &e->red_out, (size_t)ns * 8)))
         return bail(rc);
     if ((rc = apply_tiles(e))) return bail(rc);
+    if ((rc = precision == BFA_FP32 ? plan_fused<float>(e) : plan_fused<double>(e))) return bail(rc);
     if ((rc = scratch_setup(e))) return bail(rc);
     st = hipStreamSynchronize(e->stream);
     if (st != hipSuccess) {
@@ -981,6 +1005,7 @@ void bfa_destroy(bfa_env* e) {
     dfree(e->long_seg);
     dfree(e->bulk_st);
     dfree(e->bulk_ups);
+    dfree(e->xy.sm);
     for (int i = 0; i < 2; ++i) {
         if (e->aux[i]) (void)hipStreamSynchronize(e->aux[i]);
         if (e->aux[i]) (void)hipStreamDestroy(e->aux[i]);
@@ -1756,13 +1781,14 @@ int bfa_time_kernels(bfa_env* e, double dt, int reps, double* ms) {
     int rc = ready(e, dt);
     if (rc) return rc;
     const bool slabs = e->slab > 0 && e->R == 0;
+    const bool fused = !slabs && fused_active(e);
     hipEvent_t ev[6];
     for (auto& x : ev) HIP_TRY(e, hipEventCreate(&x));
     double acc[5] = {0, 0, 0, 0, 0};
     for (int r = 0; r < reps && rc == BFA_OK; ++r) {
         (void)hipEventRecord(ev[0], e->stream);
-        if (slabs) {
-            rc = enqueue_xy_slabs(e);
+        if (slabs || fused) {
+            rc = slabs ? enqueue_xy_slabs(e) : launch_fused_xy(e, e->stream, 0, e->ns, 0, e->nz);
             (void)hipEventRecord(ev[1], e->stream);
             (void)hipEventRecord(ev[2], e->stream);
             if (rc == BFA_OK) rc = launch_sweep_any(e, 2);

@@ -1,0 +1,87 @@
+"""GPU: the fused x + y sweep of the default schedule against the CPU oracle and
+against the separate sweeps, which run when kernel shapes are set explicitly.
+
+Bars: relative max-norm 1e-12 (FP64) and 1e-5 (FP32) against the oracle after
+every step, as for the separate sweeps; between the two schedules, which run
+the same recurrences and differ in the length of the x chunks, 1e-13 and 2e-6
+(the batched solver's bar for its two schedules).
+"""
+import numpy as np
+import pytest
+
+import oracle
+from helpers import agents_for, gpu_env, load_pkg, make_problem, relmax
+
+pytestmark = pytest.mark.gpu
+
+TOL = {"fp64": 1e-12, "fp32": 1e-5}
+SAME = {"fp64": 1e-13, "fp32": 2e-6}
+
+
+@pytest.fixture(scope="module")
+def pkg():
+    return load_pkg()
+
+
+def compare(pkg, shape, precision, dirichlet, solver, steps=3):
+    p = make_problem(*shape, seed=sum(shape) + 3, n_agents=40, dirichlet=dirichlet, collide=4)
+    orc = oracle.Oracle(p.nx, p.ny, p.nz, p.ns, p.dx, p.D, p.decay, p.active, p.reg, p.fv, solver=solver)
+    ag = agents_for(p)
+    u = p.u0.copy()
+    fused, sep = gpu_env(pkg, p, precision), gpu_env(pkg, p, precision)
+    try:
+        sep.set_tiles(*sep.tiles()[:3])
+        for e in (fused, sep):
+            e.set_solver(solver)
+        for _ in range(steps):
+            orc.diffusion_step(u, p.dt)
+            orc.secretion_uptake(u, ag)
+            fused.step(p.dt, 1)
+            sep.step(p.dt, 1)
+            f, s = (e.download().reshape(-1, p.ns) for e in (fused, sep))
+            ref = u.reshape(-1, p.ns)
+            for d in range(p.ns):
+                assert relmax(f[:, d], ref[:, d]) <= TOL[precision], d
+                assert relmax(f[:, d], s[:, d]) <= SAME[precision], d
+    finally:
+        fused.close()
+        sep.close()
+
+
+# one row, one column, one plane; rows of whole chunks (7, 13, 17, 25 nodes) and
+# one node either side of them; rows that are and are not whole 16-byte vectors;
+# one and several rows per wavefront; y chunks of 8 and 16 with every kind of
+# remainder; columns in one and in several passes; planes near the LDS limit
+PLANES = [(1, 5, 3, 2), (5, 1, 7, 1), (31, 17, 1, 2), (28, 16, 9, 1), (27, 33, 5, 2), (29, 32, 6, 1), (64, 63, 5, 1),
+          (100, 100, 6, 2), (101, 97, 4, 3), (257, 41, 12, 2), (453, 15, 3, 1), (12, 300, 5, 1), (203, 157, 200, 1),
+          (150, 129, 150, 1)]
+
+
+@pytest.mark.parametrize("shape", PLANES)
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_planes_match_the_oracle_and_the_separate_sweeps(pkg, shape, precision):
+    steps = 1 if np.prod(shape) > 10 ** 6 else 3
+    for dirichlet, solver in (("all", "blocking"), ("mixed", "avx256d"), ("off", "blocking")):
+        compare(pkg, shape, precision, dirichlet, solver, steps)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_windows_of_planes_are_bit_identical(pkg, precision):
+    """The slab and substrate-stream schedules sweep windows of planes and of
+    substrates; the values do not depend on the window.  Shapes that are set
+    and given back leave the default schedule as it was."""
+    p = make_problem(45, 38, 23, 3, seed=5, n_agents=30, dirichlet="mixed", collide=4)
+    out = []
+    for slab, streams, tiles in ((0, 1, False), (7, 1, False), (23, 1, False), (0, 2, False), (0, 1, True)):
+        e = gpu_env(pkg, p, precision)
+        if tiles:
+            e.set_tiles(8, 8, 8)
+            e.step(p.dt, 0)
+            e.set_tiles(0, 0, 0)
+        e.set_slab(slab)
+        e.set_substrate_streams(streams)
+        e.step(p.dt, 3)
+        out.append(e.download())
+        e.close()
+    for o in out[1:]:
+        assert np.array_equal(o, out[0])
