@@ -51,8 +51,18 @@ struct FusedPlan {
     bool on = false;
     int L = 0, LY = 0, PY = 0, W = 0, threads = 0;  // kernel shape (PlaneArgs)
     size_t lds = 0;
+    int C = 0;           // bricks per plane (0: whole planes)
     void* sm = nullptr;  // multipliers of the x scans, [ns][12][P]
+    void* A = nullptr;   // bricks: border planes (BrickBytes)
+    void* B = nullptr;
+    void* coef = nullptr;
+    void* w64 = nullptr;
+    void* zg = nullptr;
+    void* out = nullptr;
 };
+
+// Most memory that the fused sweep of one environment adds.
+constexpr size_t kBrickBytesMax = (size_t)8 << 30;
 
 struct bfa_env {
     int nx = 0, ny = 0, nz = 0, ns = 0;
@@ -589,8 +599,9 @@ int enqueue_split(bfa_env* e, bool agents) {
         const int d0 = g == 0 ? 0 : h, nd = g == 0 ? h : e->ns - h;
         const bool fused = fused_active(e);
         int rc = fused ? launch_fused_xy(e, st, d0, nd, 0, e->nz) : BFA_OK;
-        for (int a = fused ? 2 : 0; a < 3 && rc == BFA_OK; ++a)
+        for (int a = 0; a < 2 && !fused && rc == BFA_OK; ++a)
             rc = launch_sweep_win(e, a, st, Win{d0, nd, 0, axis_lines(e, a)});
+        if (rc == BFA_OK) rc = launch_z(e, st, d0, nd);
         if (rc) return rc;
         if (agents) {
             int rc = launch_agents_win(e, st, d0, nd);
@@ -729,7 +740,7 @@ int run_precompute(bfa_env* e, double dt) {
                            reinterpret_cast<T*>(e->kT), reinterpret_cast<T*>(e->betaT));
         LAUNCH_CHECK(e, "thomas precompute");
     }
-    return fused_precompute<T>(e);
+    return fused_precompute<T>(e, dt);
 }
 
 int ensure_precompute(bfa_env* e, double dt) {
@@ -780,11 +791,11 @@ int enqueue_diffusion(bfa_env* e) {
     if (e->slab > 0 && e->R == 0) {
         int rc = enqueue_xy_slabs(e);
         if (rc) return rc;
-        return launch_sweep_any(e, 2);
+        return launch_z(e, e->stream, 0, e->ns);
     }
     if (fused_active(e)) {
         int rc = launch_fused_xy(e, e->stream, 0, e->ns, 0, e->nz);
-        return rc ? rc : launch_sweep_any(e, 2);
+        return rc ? rc : launch_z(e, e->stream, 0, e->ns);
     }
     for (int a = 0; a < 3; ++a) {
         int rc = launch_sweep_any(e, a);
@@ -1005,7 +1016,7 @@ void bfa_destroy(bfa_env* e) {
     dfree(e->long_seg);
     dfree(e->bulk_st);
     dfree(e->bulk_ups);
-    dfree(e->xy.sm);
+    free_fused(e);
     for (int i = 0; i < 2; ++i) {
         if (e->aux[i]) (void)hipStreamSynchronize(e->aux[i]);
         if (e->aux[i]) (void)hipStreamDestroy(e->aux[i]);
@@ -1791,7 +1802,7 @@ int bfa_time_kernels(bfa_env* e, double dt, int reps, double* ms) {
             rc = slabs ? enqueue_xy_slabs(e) : launch_fused_xy(e, e->stream, 0, e->ns, 0, e->nz);
             (void)hipEventRecord(ev[1], e->stream);
             (void)hipEventRecord(ev[2], e->stream);
-            if (rc == BFA_OK) rc = launch_sweep_any(e, 2);
+            if (rc == BFA_OK) rc = launch_z(e, e->stream, 0, e->ns);
             (void)hipEventRecord(ev[3], e->stream);
         } else {
             for (int a = 0; a < 3 && rc == BFA_OK; ++a) {

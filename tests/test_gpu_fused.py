@@ -48,6 +48,27 @@ def compare(pkg, shape, precision, dirichlet, solver, steps=3):
         sep.close()
 
 
+# bricks of FP32 rows: 25 rows and one more or less per plane, two bricks and
+# many, whole and ragged 16-byte rows, z lines of two chunks and of several with
+# every kind of remainder, more and fewer columns than a block has threads
+BRICKS32 = [(180, 171, 26, 1), (187, 200, 50, 2), (259, 151, 51, 1), (513, 80, 33, 1), (832, 51, 74, 2), (190, 176, 75, 3),
+            (64, 700, 30, 2)]
+
+
+@pytest.mark.parametrize("shape", BRICKS32)
+def test_bricks_match_the_oracle_and_the_separate_sweeps(pkg, shape):
+    for dirichlet, solver in (("all", "blocking"), ("mixed", "avx256d"), ("mixed", "blocking"), ("off", "blocking")):
+        compare(pkg, shape, "fp32", dirichlet, solver, 2)
+
+
+@pytest.mark.parametrize("shape,precision", [((64, 801, 701), "fp64"), ((511, 270, 251), "fp64"), ((333, 401, 260), "fp64"),
+                                             ((810, 541, 77), "fp64"), ((331, 512, 501), "fp32")])
+def test_bricks_of_large_fields(pkg, shape, precision):
+    """Fields larger than the last-level cache, against the oracle: FP64 bricks
+    of 16 and 20 rows with a z block per few rows."""
+    compare(pkg, shape + (1,), precision, "all", "blocking", 1)
+
+
 # one row, one column, one plane; rows of whole chunks (7, 13, 17, 25 nodes) and
 # one node either side of them; rows that are and are not whole 16-byte vectors;
 # one and several rows per wavefront; y chunks of 8 and 16 with every kind of
@@ -65,12 +86,13 @@ def test_planes_match_the_oracle_and_the_separate_sweeps(pkg, shape, precision):
         compare(pkg, shape, precision, dirichlet, solver, steps)
 
 
-@pytest.mark.parametrize("precision", ["fp64", "fp32"])
-def test_windows_of_planes_are_bit_identical(pkg, precision):
+@pytest.mark.parametrize("shape,precision", [((45, 38, 23, 3), "fp64"), ((45, 38, 23, 3), "fp32"),
+                                             ((190, 176, 40, 3), "fp32")])
+def test_windows_of_planes_are_bit_identical(pkg, shape, precision):
     """The slab and substrate-stream schedules sweep windows of planes and of
     substrates; the values do not depend on the window.  Shapes that are set
     and given back leave the default schedule as it was."""
-    p = make_problem(45, 38, 23, 3, seed=5, n_agents=30, dirichlet="mixed", collide=4)
+    p = make_problem(*shape, seed=5, n_agents=30, dirichlet="mixed", collide=4)
     out = []
     for slab, streams, tiles in ((0, 1, False), (7, 1, False), (23, 1, False), (0, 2, False), (0, 1, True)):
         e = gpu_env(pkg, p, precision)
