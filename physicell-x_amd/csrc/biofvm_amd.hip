@@ -133,6 +133,7 @@ struct bfa_env {
     hipGraphExec_t gexec = nullptr;
     double graph_dt = -1.0;
     bool graph_valid = false;
+    bool queued = false;  // steps were launched without the graph since it was last drained
 
     int Lreq[3] = {0, 0, 0};
     int Rreq = 0;
@@ -664,12 +665,13 @@ unsigned long long face_active(const bfa_env* e) {
     return act;
 }
 
-// Drops the captured step graph.  Launches of it may still be queued or
-// running (bfa_step only enqueues them), and its kernel arguments point into
-// buffers that the caller is about to replace, so the handle's stream (which
-// every side stream joins back into) is drained first.
+// Drops the captured step graph.  Launches of it, or of a step's kernels, may
+// still be queued or running (bfa_step only enqueues them), and their arguments
+// point into buffers that the caller is about to replace, so the handle's
+// stream (which every side stream joins back into) is drained first.
 void invalidate_graph(bfa_env* e) {
-    if (e->gexec && e->stream) (void)hipStreamSynchronize(e->stream);
+    if ((e->gexec || e->queued) && e->stream) (void)hipStreamSynchronize(e->stream);
+    e->queued = false;
     if (e->gexec) (void)hipGraphExecDestroy(e->gexec);
     if (e->graph) (void)hipGraphDestroy(e->graph);
     e->gexec = nullptr;
@@ -810,6 +812,18 @@ int enqueue_step(bfa_env* e) {
     int rc = enqueue_diffusion(e);
     if (rc) return rc;
     return launch_agents(e);
+}
+
+// A step of few kernels on one stream is launched kernel by kernel: consecutive
+// graph launches left 5 us between two steps where consecutive kernels leave 1
+// to 2 (24x20x28: 18.3 us per step as a graph, 15.5 as kernels; 50^3 20.7 /
+// 17.8; 100^3 x 2 40.5 / 36.0), the host spends 11 us on a step's kernels and 14
+// on a graph, and the first call captures nothing (0.3 to 0.5 ms).  Graphs of
+// several steps replay as fast as kernels but take 0.6 to 1.7 ms to build.  The
+// slab and substrate schedules have tens of launches and events per step, which
+// a graph replays faster than the host can enqueue them.
+bool many_launches(const bfa_env* e) {
+    return e->hplanes.empty() && ((e->slab > 0 && e->R == 0) || split_schedule(e));
 }
 
 int build_graph(bfa_env* e, double dt) {
@@ -1560,6 +1574,12 @@ int bfa_step(bfa_env* e, double dt, int nsteps) {
     int rc = ready(e, dt);
     if (rc) return rc;
     if (nsteps == 0) return BFA_OK;
+    if (!many_launches(e)) {
+        e->queued = true;
+        for (int s = 0; s < nsteps; ++s)
+            if ((rc = enqueue_step(e))) return rc;
+        return BFA_OK;
+    }
     if (!e->graph_valid || e->graph_dt != dt) {
         if ((rc = build_graph(e, dt))) return rc;
     }
