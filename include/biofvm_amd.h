@@ -407,12 +407,13 @@ int bfa_batch_get_col_threads(const bfa_batch *batch, int *out2);
  * bit-identical either way.  No reference counterpart. */
 int bfa_batch_set_streams(bfa_batch *batch, int groups);
 int bfa_batch_get_streams(const bfa_batch *batch);
-/* Fused x + y sweeps (default off): members whose k-plane fits a 128 KiB
+/* Fused x + y sweeps (default on): members whose k-plane fits a 128 KiB
  * on-chip buffer are swept along x and y plane by plane in LDS, reading and
- * writing the field once for both sweeps.  Same per-line arithmetic as the
- * separate sweeps except the x chunking (5 nodes).  No reference
- * counterpart: the reference sweeps each axis over the whole grid
- * (BioFVM/BioFVM_solvers.cpp:352-730). */
+ * writing the field once for both sweeps; the x and y shapes of
+ * bfa_batch_set_tiles are those of the other members.  enabled == 0: every
+ * member takes the separate sweeps.  Same per-line arithmetic except the
+ * chunking.  No reference counterpart: the reference sweeps each axis over the
+ * whole grid (BioFVM/BioFVM_solvers.cpp:352-730). */
 int bfa_batch_set_fusion(bfa_batch *batch, int enabled);
 /* Number of live members that take the fused sweep. */
 int bfa_batch_fused_members(const bfa_batch *batch);

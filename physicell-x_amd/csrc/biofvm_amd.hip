@@ -19,8 +19,8 @@
 
 #include "biofvm_amd.h"
 #include "biofvm_aux_kernels.h"
-#include "biofvm_batch_kernels.h"
 #include "biofvm_fused_kernels.h"
+#include "biofvm_batch_kernels.h"
 #include "biofvm_kernels.h"
 #include "biofvm_transfer.inc"
 

@@ -184,18 +184,16 @@ __device__ __forceinline__ void rows_to_lds(T* tile, int S, const T* src, int nx
 }
 
 // ---- one plane per block -----------------------------------------------------------
+// Shape and tables of a plane's solve.
 template <typename T>
-struct PlaneArgs {
-    SweepArgs<T> x;      // field, x coefficients, constants, Dirichlet table, window d0
-    const T* yinv;       // [ns][ny] 1/den and c' of the y lines
+struct PlaneShape {
+    const T* yinv;  // [ns][ny] 1/den and c' of the y lines
     const T* ycp;
-    const T* sm;         // [ns][12][P] multipliers of the x scans
-    int k0;              // planes k0 .. k0 + nk.d of every substrate of the window
-    Divisor nk;
-    int P, S;            // x chunks of a row, LDS row pitch
-    int PY;              // chunks of a y column
-    int W;               // columns per pass of the y phase (W * PY <= blockDim.x)
-    int vec;             // rows are whole 16-byte vectors
+    const T* sm;    // [ns][12][P] multipliers of the x scans
+    int P, S;       // x chunks of a row, LDS row pitch
+    int PY;         // chunks of a y column
+    int W;          // columns per pass of the y phase (W * PY <= blockDim.x)
+    int vec;        // rows are whole 16-byte vectors
 };
 
 // The x sweep with the Dirichlet passes around it and the y sweep with the one
@@ -210,11 +208,9 @@ struct PlaneArgs {
 // Dynamic LDS, of T: ny*S tile | 2*roundup4(PY*LY) y coefficients | 2*P*L x
 // coefficients | 12*P scan multipliers | PY*W carries | PY products.
 template <typename T, int L, int LY, bool DEV>
-__global__ __launch_bounds__(1024) void k_sweep_xy_plane(PlaneArgs<T> g) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    const SweepArgs<T>& a = g.x;
+__device__ __forceinline__ void sweep_xy_plane(const PlaneShape<T>& g, const SweepArgs<T>& a, int d, int k, T* smem) {
     const int nx = a.nx, ny = a.ny, nz = a.nz, S = g.S, P = g.P, PY = g.PY, W = g.W;
-    T* tile = reinterpret_cast<T*>(smem);
+    T* tile = smem;
     T* s_inv = tile + ny * S;
     T* s_cp = s_inv + (PY * LY + 3) / 4 * 4;
     T* s_xi = s_cp + (PY * LY + 3) / 4 * 4;
@@ -224,9 +220,6 @@ __global__ __launch_bounds__(1024) void k_sweep_xy_plane(PlaneArgs<T> g) {
     T* s_g = s_z + PY * W;
     const int t = threadIdx.x, nthr = blockDim.x, lane = t & 63, nw = nthr >> 6;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int b = __builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x));
-    const int dd = div_by(b, g.nk);
-    const int d = a.d0 + dd, k = g.k0 + b - dd * g.nk.d;
     T* plane = a.u + (long long)d * a.N + (long long)k * ny * nx;
     if (g.vec)
         rows_to_lds<T, 16, 0>(tile, S, plane, nx, ny, wave, nw, lane);
@@ -297,6 +290,22 @@ __global__ __launch_bounds__(1024) void k_sweep_xy_plane(PlaneArgs<T> g) {
         if (act && dact) col_dirichlet<T, LY, 1>(x, a, d, i, k, sy, ny, py, PY);
         if (cnt > 0) store_line_chunk<T, LY>(x, plane + (long long)sy * nx + i, (size_t)nx, cnt);
     }
+}
+
+template <typename T>
+struct PlaneArgs {
+    SweepArgs<T> x;  // field, x coefficients, constants, Dirichlet table, window d0
+    PlaneShape<T> s;
+    int k0;          // planes k0 .. k0 + nk.d of every substrate of the window
+    Divisor nk;
+};
+
+template <typename T, int L, int LY, bool DEV>
+__global__ __launch_bounds__(1024) void k_sweep_xy_plane(PlaneArgs<T> g) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int b = __builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x));
+    const int dd = div_by(b, g.nk);
+    sweep_xy_plane<T, L, LY, DEV>(g.s, g.x, g.x.d0 + dd, g.k0 + b - dd * g.nk.d, reinterpret_cast<T*>(smem));
 }
 
 // ---- bricks of rows ------------------------------------------------------------------

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import oracle
-from helpers import agents_for, gpu_env, load_pkg, make_problem, relmax
+from helpers import agents_for, gpu_env, load_pkg, make_problem, oracle_for, relmax
 
 pytestmark = pytest.mark.gpu
 
@@ -107,3 +107,35 @@ def test_windows_of_planes_are_bit_identical(pkg, shape, precision):
         e.close()
     for o in out[1:]:
         assert np.array_equal(o, out[0])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_batch_planes_of_every_block_class(pkg, precision):
+    """Members on both sides of the limits of the batch's fused sweep: planes
+    for blocks of 256, 512 and 1024 threads, one past the plane buffer and one
+    past its column chunks, against the oracle and the separate sweeps."""
+    shapes = [(1, 1, 4, 1), (7, 16, 9, 2), (33, 17, 5, 3), (64, 75, 6, 1), (65, 131, 5, 2), (128, 128, 4, 1),
+              (160, 160, 3, 1), (181, 181, 3, 1), (16, 321, 4, 1), (18, 320, 4, 2), (512, 31, 3, 1)]
+    ps = [make_problem(*sh, seed=900 + k, n_agents=20, dirichlet=("all", "mixed", "off")[k % 3], collide=3)
+          for k, sh in enumerate(shapes)]
+    out = {}
+    for fuse in (True, False):
+        with pkg.Batch(precision) as b:
+            if not fuse:
+                b.set_fusion(False)
+            ids = []
+            for p in ps:
+                ids.append(b.add(p.nx, p.ny, p.nz, p.ns, p.dx, p.D, p.decay, p.active, p.reg, p.fv))
+                b.upload(ids[-1], p.u0)
+                b.set_agents(ids[-1], p.voxel, p.c1, p.c2, p.e2, p.agent_active)
+            b.step(ps[0].dt, 2)
+            out[fuse] = [b.download(i) for i in ids]
+    for p, f, s in zip(ps, out[True], out[False]):
+        orc, ag, u = oracle_for(p), agents_for(p), p.u0.copy()
+        for _ in range(2):
+            orc.diffusion_step(u, p.dt)
+            orc.secretion_uptake(u, ag)
+        f, s, ref = (x.reshape(-1, p.ns) for x in (f, s, u))
+        for d in range(p.ns):
+            assert relmax(f[:, d], ref[:, d]) <= TOL[precision], (p.nx, p.ny, d)
+            assert relmax(f[:, d], s[:, d]) <= SAME[precision], (p.nx, p.ny, d)
