@@ -289,7 +289,7 @@ __global__ __launch_bounds__(1024) void kb_sweep_xy(const EnvDesc<T>* __restrict
     const XYItem w = items[__builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x))];
     const EnvDesc<T>& e = envs[w.env];
     if (step >= e.steps) return;
-    sweep_xy_plane<T, L, LY, DEV>(e.xy, args_of<T>(e, 0), w.d, w.k, reinterpret_cast<T*>(smem));
+    sweep_xy_plane<T, L, LY, DEV, false>(e.xy, args_of<T>(e, 0), w.d, w.k, reinterpret_cast<T*>(smem));
 }
 
 // Agent entries over the whole batch: entry q updates the value at absolute

@@ -207,7 +207,7 @@ struct PlaneShape {
 // 89.4 -> 78.9 us.
 // Dynamic LDS, of T: ny*S tile | 2*roundup4(PY*LY) y coefficients | 2*P*L x
 // coefficients | 12*P scan multipliers | PY*W carries | PY products.
-template <typename T, int L, int LY, bool DEV>
+template <typename T, int L, int LY, bool DEV, bool PV>
 __device__ __forceinline__ void sweep_xy_plane(const PlaneShape<T>& g, const SweepArgs<T>& a, int d, int k, T* smem) {
     const int nx = a.nx, ny = a.ny, nz = a.nz, S = g.S, P = g.P, PY = g.PY, W = g.W;
     T* tile = smem;
@@ -240,15 +240,26 @@ __device__ __forceinline__ void sweep_xy_plane(const PlaneShape<T>& g, const Swe
     }
     const bool dact = (a.active >> d) & 1ull;
     const T kd = a.k[d], lam = DEV ? a.k[a.ns + d] : T(0), bt = DEV ? a.beta[d] : T(0);
-    const T v_lo = a.dval[dir_slot_xonly(0, nx, a.reg) * a.ns + d];
-    const T v_hi = a.dval[dir_slot_xonly(nx - 1, nx, a.reg) * a.ns + d];
+    const T v_lo = PV ? T(0) : a.dval[dir_slot_xonly(0, nx, a.reg) * a.ns + d];
+    const T v_hi = PV ? T(0) : a.dval[dir_slot_xonly(nx - 1, nx, a.reg) * a.ns + d];
+    // Dirichlet value of a boundary voxel of this plane
+    auto value = [&](int i, int j) {
+        return PV ? dir_value(a, d, i, j, k) : a.dval[dir_slot(i, j, k, nx, ny, nz, a.reg) * a.ns + d];
+    };
     const int RW = 64 / P, rw = lane / P, p = rw < RW ? lane - rw * P : 0;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's rows are in LDS
     __syncthreads();
+    if (PV && dact) {  // the row ends differ from row to row
+        for (int e = t; e < 2 * ny; e += nthr) {
+            const int r = e >> 1, i = e & 1 ? nx - 1 : 0;
+            tile[r * S + i] = value(i, r);
+        }
+        __syncthreads();
+    }
     // x phase.  Rows on a y or z face are solved too and overwritten below.
     for (int r = wave * RW; r < ny; r += nw * RW) {
         const bool on = rw < RW && r + rw < ny;
-        lds_row_solve<T, L, DEV>(tile + (on ? r + rw : r) * S, on, nx, p, P, dact, v_lo, v_hi, s_xi, s_xc, s_sm, kd, lam,
+        lds_row_solve<T, L, DEV>(tile + (on ? r + rw : r) * S, on, nx, p, P, dact && !PV, v_lo, v_hi, s_xi, s_xc, s_sm, kd, lam,
                                  bt);
     }
     __syncthreads();
@@ -267,8 +278,8 @@ __device__ __forceinline__ void sweep_xy_plane(const PlaneShape<T>& g, const Swe
         const bool ends = act && dact && !kface && i > 0 && i < nx - 1;
         T vlast = T(0);
         if (ends) {
-            vlast = a.dval[dir_slot(i, ny - 1, k, nx, ny, nz, a.reg) * a.ns + d];
-            if (sy == 0) x[0] = a.dval[dir_slot(i, 0, k, nx, ny, nz, a.reg) * a.ns + d];
+            vlast = value(i, ny - 1);
+            if (sy == 0) x[0] = value(i, 0);
             if (cnt <= LY) {
 #pragma unroll
                 for (int m = 0; m < LY; ++m)
@@ -287,7 +298,14 @@ __device__ __forceinline__ void sweep_xy_plane(const PlaneShape<T>& g, const Swe
 #pragma unroll
             for (int m = 0; m < LY; ++m) x[m] = (m < cnt ? col[m * S] : T(0)) + x[m];
         }
-        if (act && dact) col_dirichlet<T, LY, 1>(x, a, d, i, k, sy, ny, py, PY);
+        if (PV && act && dact) {
+            const bool whole = kface || i == 0 || i == nx - 1;
+#pragma unroll
+            for (int m = 0; m < LY; ++m)
+                if (m < cnt && (whole || sy + m == 0 || m == cnt - 1)) x[m] = value(i, sy + m);
+        } else if (act && dact) {
+            col_dirichlet<T, LY, 1>(x, a, d, i, k, sy, ny, py, PY);
+        }
         if (cnt > 0) store_line_chunk<T, LY>(x, plane + (long long)sy * nx + i, (size_t)nx, cnt);
     }
 }
@@ -300,12 +318,14 @@ struct PlaneArgs {
     Divisor nk;
 };
 
-template <typename T, int L, int LY, bool DEV>
+// PV: the Dirichlet values are per-voxel planes (SweepArgs::plane), which the
+// separate sweeps need four face passes of their own for.
+template <typename T, int L, int LY, bool DEV, bool PV>
 __global__ __launch_bounds__(1024) void k_sweep_xy_plane(PlaneArgs<T> g) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int b = __builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x));
     const int dd = div_by(b, g.nk);
-    sweep_xy_plane<T, L, LY, DEV>(g.s, g.x, g.x.d0 + dd, g.k0 + b - dd * g.nk.d, reinterpret_cast<T*>(smem));
+    sweep_xy_plane<T, L, LY, DEV, PV>(g.s, g.x, g.x.d0 + dd, g.k0 + b - dd * g.nk.d, reinterpret_cast<T*>(smem));
 }
 
 // ---- bricks of rows ------------------------------------------------------------------

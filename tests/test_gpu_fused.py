@@ -139,3 +139,27 @@ def test_batch_planes_of_every_block_class(pkg, precision):
         for d in range(p.ns):
             assert relmax(f[:, d], ref[:, d]) <= TOL[precision], (p.nx, p.ny, d)
             assert relmax(f[:, d], s[:, d]) <= SAME[precision], (p.nx, p.ny, d)
+
+
+@pytest.mark.parametrize("shape", [(1, 5, 3, 2), (5, 1, 7, 1), (31, 17, 1, 2), (29, 33, 6, 3), (64, 63, 5, 1), (257, 41, 12, 2),
+                                   (12, 300, 5, 1), (128, 96, 20, 1)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_per_voxel_dirichlet_planes(pkg, shape, precision):
+    """Values that vary along the faces, on both schedules and both solvers."""
+    nx, ny, nz, ns = shape
+    for dirichlet, solver in (("all", "blocking"), ("mixed", "avx256d")):
+        p = make_problem(*shape, seed=sum(shape) + 11, n_agents=20, dirichlet=dirichlet, collide=3)
+        v = np.random.default_rng(sum(shape)).uniform(0, 40, (nx, ny, nz, ns))
+        planes = [v[0], v[-1], v[:, 0], v[:, -1], v[:, :, 0], v[:, :, -1]]
+        out = []
+        for separate in (False, True):
+            e = gpu_env(pkg, p, precision)
+            if separate:
+                e.set_tiles(*e.tiles()[:3])
+            e.set_solver(solver)
+            e.set_dirichlet_planes(planes)
+            e.step(p.dt, 3)
+            out.append(e.download().reshape(-1, ns))
+            e.close()
+        for d in range(ns):
+            assert relmax(out[0][:, d], out[1][:, d]) <= SAME[precision], (solver, d)
