@@ -52,7 +52,7 @@ def compare(pkg, shape, precision, dirichlet, solver, steps=3):
 # many, whole and ragged 16-byte rows, z lines of two chunks and of several with
 # every kind of remainder, more and fewer columns than a block has threads
 BRICKS32 = [(180, 171, 26, 1), (187, 200, 50, 2), (259, 151, 51, 1), (513, 80, 33, 1), (832, 51, 74, 2), (190, 176, 75, 3),
-            (64, 700, 30, 2)]
+            (120, 400, 30, 2)]
 
 
 @pytest.mark.parametrize("shape", BRICKS32)
