@@ -177,8 +177,8 @@ int bfa_diffusion_decay(bfa_env *env, double dt);
  * bfa_set_agents, composed per voxel in ascending agent order. */
 int bfa_secretion_uptake(bfa_env *env);
 /* nsteps x (bfa_diffusion_decay(dt); bfa_secretion_uptake), enqueued on the
- * handle's stream (schedules of many launches per step as a captured HIP
- * graph). */
+ * handle's stream (large fields and schedules of many launches per step as a
+ * captured HIP graph). */
 int bfa_step(bfa_env *env, double dt, int nsteps);
 /* apply_dirichlet_boundaries_conditions on the resident field. */
 int bfa_apply_dirichlet(bfa_env *env);

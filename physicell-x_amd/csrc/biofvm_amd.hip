@@ -893,8 +893,14 @@ int enqueue_step(bfa_env* e) {
 // on a graph, and the first call captures nothing (0.3 to 0.5 ms).  Graphs of
 // several steps replay as fast as kernels but take 0.6 to 1.7 ms to build.  The
 // slab and substrate schedules have tens of launches and events per step, which
-// a graph replays faster than the host can enqueue them.
-bool many_launches(const bfa_env* e) {
+// a graph replays faster than the host can enqueue them.  Fields above 40 MiB
+// keep the graph too: their steps take 60 us and more, and hundreds of kernels
+// enqueued ahead made a program with busy host threads unsteady (203x157x121 x
+// 3 FP32, 100 steps and a save in single precision: 9.7 to 9.9 ms as graphs,
+// 10.3 to 11.9 as kernels over eleven runs; 131x257x67 x 2 FP64, 34 MiB: 7.6 as
+// graphs, 7.2 as kernels).
+bool step_as_graph(const bfa_env* e) {
+    if ((size_t)e->N * e->ns * e->tsize > (size_t)40 << 20) return true;
     return e->hplanes.empty() && ((e->slab > 0 && e->R == 0) || split_schedule(e));
 }
 
@@ -1647,7 +1653,7 @@ int bfa_step(bfa_env* e, double dt, int nsteps) {
     int rc = ready(e, dt);
     if (rc) return rc;
     if (nsteps == 0) return BFA_OK;
-    if (!many_launches(e)) {
+    if (!step_as_graph(e)) {
         e->queued = true;
         for (int s = 0; s < nsteps; ++s)
             if ((rc = enqueue_step(e))) return rc;
