@@ -19,7 +19,9 @@ sweep kernels on the GPU (HIP events around each launch, via
 * schedule: whole-volume sweeps, the two substrate halves swept on parallel
   streams, or (FP64) x/y sweeps in k-slabs of a few planes, the slabs with
   each of the three fastest wave x chunk lengths (chosen by graph-replayed
-  whole-step time; slabs have to win by 2 %).
+  whole-step time; slabs have to win by 2 %);
+* the library's default schedule, which may sweep x and y together: it is
+  kept, as shapes of 0, when its whole step is the fastest.
 
 Results are cached per (nx, ny, nz, ns, precision) in memory and, when a path
 is given, in a JSON file.
@@ -213,6 +215,23 @@ def autotune(pkg, nx, ny, nz, ns, precision="fp32", dt=0.01, reps=6, cache_path=
                "ms": {"x": wave_best[best_sched[3]][0] if best_sched[3] != best_x[1] else best_grid[0],
                       "y": best_ry[0], "z": best_rz[0], "step": best_sched[0]},
                "trials": trials}
+        # the default schedule (400^3 x 4: 1.00 ms FP32 and 1.68 ms FP64 against
+        # 1.22 and 2.18 with the best separate sweeps)
+        try:
+            env.set_tiles(0, 0, 0, 0, 0, 0)
+            default = True
+        except Exception:
+            default = False
+        if default:
+            env.set_x_grid(0)
+            env.set_col_runs(1, 1)
+            t = _step_ms(env, dt, reps)
+            trials.append({"axis": "schedule", "default": True, "ms_step": t})
+            if t < best_sched[0]:
+                ms = env.time_kernels(dt, reps)
+                res.update({"Lx": 0, "rows_x": 0, "Ly": 0, "cols_y": 0, "Lz": 0, "cols_z": 0, "x_grid": 0,
+                            "runs_y": 1, "runs_z": 1, "slab": 0, "substrate_streams": 1,
+                            "ms": {"x": ms[0], "y": ms[1], "z": ms[2], "step": t}})
     finally:
         env.close()
     if verbose:
