@@ -201,10 +201,10 @@ struct PlaneShape {
 // per wavefront (lds_row_solve).  y: PY threads per column, W columns at a
 // time, chunk_solve as the separate sweep.  What bounds it on small and middle
 // grids is the chain load - x - y - store of one block per CU, so the block
-// takes as many threads as both phases can use (plan_fused).  Measured (step,
-// separate sweeps -> this): 50^3 FP64 23.2 -> 20.0 us, 75^3 x 2 FP32 28.7 ->
-// 22.7, 100^3 x 2 FP64 50.2 -> 39.1, FP32 39.4 -> 29.0, 203x157x121 x 3 FP32
-// 89.4 -> 78.9 us.
+// takes as many threads as both phases can use (plan_planes).  Measured (step,
+// separate sweeps -> this): 50^3 FP64 22.7 -> 14.3 us, 75^3 x 2 FP32 24.8 ->
+// 18.8, 100^3 x 2 FP64 45.8 -> 34.4, FP32 35.0 -> 24.3, 203x157x121 x 3 FP32
+// 89.4 -> 74.9 us.
 // Dynamic LDS, of T: ny*S tile | 2*roundup4(PY*LY) y coefficients | 2*P*L x
 // coefficients | 12*P scan multipliers | PY*W carries | PY products.
 template <typename T, int L, int LY, bool DEV, bool PV>
@@ -259,8 +259,8 @@ __device__ __forceinline__ void sweep_xy_plane(const PlaneShape<T>& g, const Swe
     // x phase.  Rows on a y or z face are solved too and overwritten below.
     for (int r = wave * RW; r < ny; r += nw * RW) {
         const bool on = rw < RW && r + rw < ny;
-        lds_row_solve<T, L, DEV>(tile + (on ? r + rw : r) * S, on, nx, p, P, dact && !PV, v_lo, v_hi, s_xi, s_xc, s_sm, kd, lam,
-                                 bt);
+        lds_row_solve<T, L, DEV>(tile + (on ? r + rw : r) * S, on, nx, p, P, dact && !PV, v_lo, v_hi, s_xi, s_xc,
+                                 s_sm, kd, lam, bt);
     }
     __syncthreads();
     // y phase: thread (yi, py) owns rows [py*LY, py*LY + LY) of column c0 + yi
