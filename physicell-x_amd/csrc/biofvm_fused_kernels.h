@@ -65,8 +65,9 @@ __device__ __forceinline__ double lane_get(double v, int from) {
 // tested for its place in the row: the Dirichlet ends are set in LDS first,
 // coefficients past the row end are zero (so the padding solves to zero), and
 // the first padded node repeats the last one, which makes the FP32 form's link
-// past the row end vanish.  Lanes without a row (on false) solve the row that
-// `row` points to and do not store.
+// past the row end vanish.  Lanes without a row (on false) solve the values that
+// `row` points to and do not store; these have to be finite, since a scan step
+// that is off still multiplies another row's value by zero.
 template <typename T, int L, bool DEV>
 __device__ __forceinline__ void lds_row_solve(T* __restrict__ row, bool on, int nx, int p, int P, bool dact, T v_lo,
                                               T v_hi, const T* __restrict__ s_xi, const T* __restrict__ s_xc,
@@ -256,11 +257,15 @@ __device__ __forceinline__ void sweep_xy_plane(const PlaneShape<T>& g, const Swe
         }
         __syncthreads();
     }
-    // x phase.  Rows on a y or z face are solved too and overwritten below.
+    // x phase.  Held rows on a y face are left out: the Dirichlet passes set them
+    // below whatever they hold, and a NaN or infinity there would reach the rows
+    // that share the wavefront.  Held planes are solved too and overwritten whole.
+    const int jlo = dact ? 1 : 0, jhi = dact ? ny - 1 : ny;
     for (int r = wave * RW; r < ny; r += nw * RW) {
-        const bool on = rw < RW && r + rw < ny;
-        lds_row_solve<T, L, DEV>(tile + (on ? r + rw : r) * S, on, nx, p, P, dact && !PV, v_lo, v_hi, s_xi, s_xc,
-                                 s_sm, kd, lam, bt);
+        const int j = r + rw;
+        const bool on = rw < RW && j >= jlo && j < jhi;
+        lds_row_solve<T, L, DEV>(on ? tile + j * S : s_xi, on, nx, p, P, dact && !PV, v_lo, v_hi, s_xi, s_xc, s_sm, kd,
+                                 lam, bt);
     }
     __syncthreads();
     // y phase: thread (yi, py) owns rows [py*LY, py*LY + LY) of column c0 + yi
@@ -635,10 +640,11 @@ __global__ __launch_bounds__(1024) void k_sweep_xy_brick(BrickArgs<T> g) {
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's rows are in LDS
     __syncthreads();
-    // x phase: RW rows per wavefront
+    // x phase: RW rows per wavefront, held rows left out as in sweep_xy_plane
+    const int rlo = dact && j0 == 0 ? 1 : 0, rhi = dact && j1 == ny ? nrx - 1 : nrx;
     for (int r = wave * RW; r < nrx; r += nw * RW) {
-        const bool on = rw < RW && r + rw < nrx;
-        lds_row_solve<T, L, DEV>(tile + (on ? r + rw : r) * S, on, nx, p, P, dact, v_lo, v_hi, s_xi, s_xc, s_sm, kd, lam,
+        const bool on = rw < RW && r + rw >= rlo && r + rw < rhi;
+        lds_row_solve<T, L, DEV>(on ? tile + (r + rw) * S : s_xi, on, nx, p, P, dact, v_lo, v_hi, s_xi, s_xc, s_sm, kd, lam,
                                  bt);
     }
     __syncthreads();
