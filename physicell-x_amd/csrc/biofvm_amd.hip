@@ -376,6 +376,15 @@ int choose_tiles(bfa_env* e) {
     return BFA_OK;
 }
 
+// Dynamic LDS up to the device's limit for a kernel.  The limit belongs to the
+// kernel, which every environment shares: set to one environment's need, it
+// would fall below what another one launches with.
+bool allow_lds(const bfa_env* e, const void* fn) {
+    if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, e->max_lds) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
 template <typename T>
 int raise_lds_limits(bfa_env* e);
 
@@ -541,9 +550,8 @@ int raise_lds_limits(bfa_env* e) {
                             lds_col(e, e->nz, e->L[2], e->TX[2])};
     const void* fn[3] = {fx, fy, fz};
     for (int a = 0; a < 3; ++a)
-        if (need[a] > 65536 && fn[a])
-            HIP_TRY(e, hipFuncSetAttribute(fn[a], hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)need[a]));
+        if (need[a] > 65536 && fn[a] && !allow_lds(e, fn[a]))
+            return fail(e, BFA_ERR_HIP, "axis %d: %zu bytes of LDS refused", a, need[a]);
     if (e->R == 0) {
         const void* fw = nullptr;
         const void* fwr = nullptr;
