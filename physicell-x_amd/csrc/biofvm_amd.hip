@@ -49,6 +49,7 @@ constexpr size_t kFieldSlack = 64;
 // (biofvm_fused_host.inc): fixed by its grid and precision.
 struct FusedPlan {
     bool on = false;
+    bool ready = false;  // the tables hold the current coefficients
     int L = 0, LY = 0, PY = 0, W = 0, threads = 0;  // kernel shape (PlaneArgs)
     size_t lds = 0;
     int C = 0;           // bricks per plane (0: whole planes)
@@ -189,10 +190,17 @@ int fail(bfa_env* e, int code, const char* fmt, ...) {
             return fail((e), BFA_ERR_HIP, "launch of %s failed: %s", what, hipGetErrorString(_st)); \
     } while (0)
 
+// Gives up the memory that a handle only keeps for speed; false if it had none.
+bool reclaim(bfa_env* e);
+
 template <typename P>
 int dalloc(bfa_env* e, P** p, size_t bytes) {
     void* q = nullptr;
     hipError_t st = hipMalloc(&q, bytes ? bytes : 16);
+    if (st != hipSuccess && reclaim(e)) {
+        (void)hipGetLastError();
+        st = hipMalloc(&q, bytes ? bytes : 16);
+    }
     if (st != hipSuccess) {
         (void)hipGetLastError();
         return fail(e, BFA_ERR_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(st));
@@ -629,7 +637,23 @@ unsigned long long face_active(const bfa_env* e) {
     return act;
 }
 
+void invalidate_graph(bfa_env* e);
+
 #include "biofvm_fused_host.inc"
+
+// Kept agent blocks, and the memory of the fused sweep: the handle runs the
+// separate sweeps from then on.
+bool reclaim(bfa_env* e) {
+    const bool any = !e->spare.empty() || e->xy.sm;
+    free_spare(e);
+    if (e->xy.sm) {
+        invalidate_graph(e);
+        (void)hipStreamSynchronize(e->stream);
+        free_fused(e);
+        e->xy.on = false;
+    }
+    return any;
+}
 
 // x and y sweeps in k-slabs of e->slab planes, per substrate, alternating
 // between two side streams so the x sweep of one slab overlaps the y sweep of
@@ -820,7 +844,12 @@ int run_precompute(bfa_env* e, double dt) {
 int ensure_precompute(bfa_env* e, double dt) {
     if (!e->coef_set) return fail(e, BFA_ERR_STATE, "bfa_set_coefficients has not been called");
     if (!(dt > 0.0) || !std::isfinite(dt)) return fail(e, BFA_ERR_ARG, "dt must be positive, got %g", dt);
-    if (e->pre_valid && (e->pre_dt == dt || e->keep_first_dt)) return BFA_OK;
+    if (e->pre_valid && (e->pre_dt == dt || e->keep_first_dt)) {
+        if (e->xy.ready || !fused_active(e)) return BFA_OK;
+        // the fused sweep runs again: its tables for the coefficients in use
+        invalidate_graph(e);
+        return e->prec == BFA_FP32 ? fused_precompute<float>(e, e->pre_dt) : fused_precompute<double>(e, e->pre_dt);
+    }
     invalidate_graph(e);
     int rc = e->prec == BFA_FP32 ? run_precompute<float>(e, dt) : run_precompute<double>(e, dt);
     if (rc) return rc;
@@ -1076,7 +1105,10 @@ int bfa_create(bfa_env** out, int nx, int ny, int nz, int ns, double dx, int pre
         (rc = dalloc(e, &e->red_out, (size_t)ns * 8)))
         return bail(rc);
     if ((rc = apply_tiles(e))) return bail(rc);
-    if ((rc = precision == BFA_FP32 ? plan_fused<float>(e) : plan_fused<double>(e))) return bail(rc);
+    if (precision == BFA_FP32)
+        plan_fused<float>(e);
+    else
+        plan_fused<double>(e);
     if ((rc = scratch_setup(e))) return bail(rc);
     st = hipStreamSynchronize(e->stream);
     if (st != hipSuccess) {
@@ -1225,6 +1257,7 @@ int bfa_set_dirichlet_planes(bfa_env* e, const double* planes) {
     e->shell = shell;
     e->hplanes.swap(h);
     e->pre_valid = false;
+    drop_unused_fused(e);
     return BFA_OK;
 }
 
@@ -2090,6 +2123,7 @@ int bfa_set_tiles(bfa_env* e, int Lx, int Ly, int Lz, int rows_x, int cols_y, in
     }
     if (e->R != 0) e->slab = 0;
     invalidate_graph(e);
+    drop_unused_fused(e);
     return BFA_OK;
 }
 
