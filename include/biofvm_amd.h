@@ -272,6 +272,12 @@ int bfa_copy_kernel_stream(size_t bytes, int reps, double *ms);
  * kept.  bfa_get_tiles writes {Lx, Ly, Lz, rows_x, cols_y, cols_z}. */
 int bfa_set_tiles(bfa_env *env, int Lx, int Ly, int Lz, int rows_x, int cols_y, int cols_z);
 int bfa_get_tiles(const bfa_env *env, int *out6);
+/* The x and y sweeps that the next step runs: out6 = {form, x chunk, y chunk,
+ * columns per pass or bricks per plane, threads per block, dynamic LDS in
+ * bytes}, form 0: separate sweeps (the rest 0), 1: whole k-planes, 2: bricks of
+ * rows.  Bricks may still turn into separate sweeps in the first step, for want
+ * of device memory. */
+int bfa_get_schedule(const bfa_env *env, int *out6);
 
 /* Sweep schedule.  planes == 0: each sweep covers the whole volume.
  * planes > 0: the x and y sweeps run in slabs of `planes` k-planes per

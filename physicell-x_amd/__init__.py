@@ -90,6 +90,7 @@ def lib():
     L.bfa_copy_kernel_stream.argtypes = [ctypes.c_size_t, ctypes.c_int, _dp]
     L.bfa_set_tiles.argtypes = [_vp] + [ctypes.c_int] * 6
     L.bfa_get_tiles.argtypes = [_vp, ctypes.POINTER(ctypes.c_int)]
+    L.bfa_get_schedule.argtypes = [_vp, ctypes.POINTER(ctypes.c_int)]
     L.bfa_set_slab.argtypes = [_vp, ctypes.c_int]
     L.bfa_get_slab.argtypes = [_vp]
     L.bfa_batch_create.argtypes = [P, ctypes.c_int]
@@ -315,6 +316,14 @@ class Microenvironment:
         v = (ctypes.c_int * 6)()
         self._check(lib().bfa_get_tiles(self._h, v), "get_tiles")
         return tuple(v)
+
+    def schedule(self):
+        """The x and y sweeps of the next step: ("separate",), ("planes", x chunk,
+        y chunk, columns per pass, threads, LDS bytes) or ("bricks", x chunk, rows,
+        bricks per plane, threads, LDS bytes)."""
+        v = (ctypes.c_int * 6)()
+        self._check(lib().bfa_get_schedule(self._h, v), "get_schedule")
+        return (("separate", "planes", "bricks")[v[0]],) + (tuple(v)[1:] if v[0] else ())
 
     def set_slab(self, planes):
         """x/y sweeps in k-slabs of `planes` planes (0: whole-volume sweeps)."""

@@ -2138,6 +2138,16 @@ int bfa_get_tiles(const bfa_env* e, int* out6) {
     return BFA_OK;
 }
 
+int bfa_get_schedule(const bfa_env* e, int* out6) {
+    if (!e || !out6) return BFA_ERR_ARG;
+    std::fill(out6, out6 + 6, 0);
+    if (!fused_active(e)) return BFA_OK;
+    const FusedPlan& q = e->xy;
+    const int v[6] = {q.C ? 2 : 1, q.L, q.LY, q.C ? q.C : q.W, q.threads, (int)q.lds};
+    std::copy(v, v + 6, out6);
+    return BFA_OK;
+}
+
 }  // extern "C"
 
 // ---- batches of independent microenvironments ------------------------------

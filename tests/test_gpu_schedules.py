@@ -5,7 +5,8 @@ import ctypes
 import numpy as np
 import pytest
 
-from helpers import agents_for, gpu_env, load_pkg, make_problem, oracle_for, relmax
+from helpers import gpu_env, load_pkg, make_problem, oracle_for, relmax
+from test_gpu_fused import SAME, compare
 
 pytestmark = pytest.mark.gpu
 
@@ -111,3 +112,102 @@ def test_memory_of_the_fused_sweep_is_held_while_it_runs(pkg):
         for x in (e, sep, pv):
             x.close()
     assert used() < field
+
+
+def planned(pkg, shape, precision):
+    e = pkg.Microenvironment(*shape, 20.0, precision)
+    try:
+        return e.schedule()
+    finally:
+        e.close()
+
+
+# whole planes: every kernel (x chunk, y chunk) that the plan can choose, with
+# columns in one pass and, third entry set, in several; the last of each
+# precision near the LDS limit
+PLANES = [("fp64", (33, 17, 7, 2), (7, 8), 0), ("fp64", (257, 1, 267, 2), (7, 8), 1), ("fp64", (1, 73, 1, 1), (7, 16), 0),
+          ("fp64", (24, 74, 9, 2), (7, 16), 0), ("fp64", (146, 127, 78, 2), (7, 16), 1), ("fp64", (328, 19, 3, 1), (13, 8), 0),
+          ("fp64", (518, 1, 260, 1), (13, 8), 1), ("fp64", (551, 9, 1, 1), (13, 16), 0), ("fp64", (128, 96, 112, 1), (13, 16), 0),
+          ("fp64", (262, 9, 549, 1), (13, 16), 1), ("fp64", (522, 18, 54, 1), (17, 8), 1), ("fp64", (425, 17, 7, 2), (17, 16), 0),
+          ("fp64", (515, 26, 40, 2), (17, 16), 1), ("fp64", (501, 28, 12, 3), (17, 16), 0),
+          ("fp32", (33, 17, 7, 2), (7, 8), 0), ("fp32", (266, 1, 526, 1), (7, 8), 1), ("fp32", (24, 74, 9, 2), (7, 16), 0),
+          ("fp32", (450, 2, 3, 1), (13, 8), 0), ("fp32", (519, 1, 260, 1), (13, 8), 1), ("fp32", (520, 9, 1, 1), (13, 16), 0),
+          ("fp32", (128, 96, 112, 1), (13, 16), 0), ("fp32", (257, 9, 275, 2), (13, 16), 1), ("fp32", (533, 17, 8, 3), (17, 8), 1),
+          ("fp32", (421, 17, 1, 1), (17, 16), 0), ("fp32", (535, 25, 60, 1), (17, 16), 1), ("fp32", (569, 17, 15, 3), (25, 8), 1),
+          ("fp32", (88, 163, 50, 1), (25, 16), 0), ("fp32", (775, 19, 36, 2), (25, 16), 1), ("fp32", (507, 62, 35, 3), (17, 16), 1)]
+
+
+@pytest.mark.parametrize("precision,shape,kernel,passes", PLANES)
+def test_planes_of_every_kernel(pkg, precision, shape, kernel, passes):
+    s = planned(pkg, shape, precision)
+    assert s[0] == "planes" and s[1:3] == kernel and (s[3] < shape[0]) == bool(passes), s
+    for dirichlet, solver in (("all", "blocking"), ("mixed", "avx256d")):
+        compare(pkg, shape, precision, dirichlet, solver, 1 if np.prod(shape) > 10 ** 6 else 2)
+
+
+def test_the_plane_cases_reach_the_lds_limit(pkg):
+    for precision in ("fp64", "fp32"):
+        assert max(planned(pkg, sh, p)[5] for p, sh, *_ in PLANES if p == precision) > 128 << 10
+
+
+@pytest.mark.parametrize("precision,shape,kernel,passes", PLANES)
+def test_per_voxel_planes_of_every_kernel(pkg, precision, shape, kernel, passes):
+    """Against the separate sweeps with their face passes."""
+    nx, ny, nz, ns = shape
+    p = make_problem(*shape, seed=sum(shape) + 17, dirichlet="mixed")
+    v = np.random.default_rng(sum(shape)).uniform(0, 40, (nx, ny, nz, ns))
+    planes = [v[0], v[-1], v[:, 0], v[:, -1], v[:, :, 0], v[:, :, -1]]
+    out = []
+    for separate in (False, True):
+        e = gpu_env(pkg, p, precision)
+        if separate:
+            e.set_tiles(*e.tiles()[:3])
+        e.set_dirichlet_planes(planes)
+        assert e.schedule()[0] == ("separate" if separate else "planes")
+        e.step(p.dt, 2)
+        out.append(e.download().reshape(-1, ns))
+        e.close()
+    for d in range(ns):
+        assert relmax(out[0][:, d], out[1][:, d]) <= SAME[precision], d
+
+
+# 17 to 32 bricks per plane and more, and few of long rows; a middle field swept by plane
+@pytest.mark.parametrize("shape,bricks", [((121, 426, 30, 1), 18), ((120, 830, 27, 1), 34), ((820, 51, 74, 2), 3),
+                                          ((203, 157, 121, 3), 0)])
+def test_fp32_bricks_and_planes_of_middle_fields(pkg, shape, bricks):
+    s = planned(pkg, shape, "fp32")
+    assert s[0] == ("bricks" if bricks else "planes") and (not bricks or s[3] == bricks), s
+    compare(pkg, shape, "fp32", "mixed", "avx256d", 1)
+
+
+# FP64 bricks of 20 and 16 rows, one block of 256, 512 and 1024 threads
+@pytest.mark.parametrize("shape,rows,threads", [((150, 130, 450, 4), 20, 256), ((333, 90, 300, 4), 20, 512),
+                                                ((500, 110, 170, 4), 16, 512), ((600, 70, 210, 4), 20, 1024)])
+@pytest.mark.parametrize("dirichlet,solver", [("mixed", "avx256d"), ("mixed", "blocking"), ("off", "blocking")])
+def test_fp64_bricks_with_free_faces_and_windows(pkg, shape, rows, threads, dirichlet, solver):
+    """Against the separate sweeps; k-slabs, substrate streams and z tile runs
+    give the same values bit for bit."""
+    p = make_problem(*shape, seed=sum(shape), n_agents=50, dirichlet=dirichlet, collide=4)
+
+    def run(setting):
+        e = gpu_env(pkg, p, "fp64")
+        e.set_solver(solver)
+        setting(e)
+        s = e.schedule()
+        e.step(p.dt, 2)
+        u = e.download().reshape(-1, p.ns)
+        e.close()
+        return s, u
+
+    s, u = run(lambda e: None)
+    assert s[0] == "bricks" and s[2] == rows and s[4] == threads, s
+    assert np.isfinite(u).all()
+    s, v = run(lambda e: e.set_tiles(*e.tiles()[:3]))
+    assert s == ("separate",)
+    for d in range(p.ns):
+        assert relmax(u[:, d], v[:, d]) <= SAME["fp64"], d
+    if solver == "avx256d":
+        for setting in (lambda e: e.set_slab(71), lambda e: e.set_substrate_streams(2), lambda e: e.set_col_runs(1, 5)):
+            s, v = run(setting)
+            assert s[0] == "bricks"
+            assert np.array_equal(u, v)
