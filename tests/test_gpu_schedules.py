@@ -211,3 +211,15 @@ def test_fp64_bricks_with_free_faces_and_windows(pkg, shape, rows, threads, diri
             s, v = run(setting)
             assert s[0] == "bricks"
             assert np.array_equal(u, v)
+
+
+# fields from HBM on both sides of the lines of bricks_lose
+@pytest.mark.parametrize("precision,shape,form", [
+    ("fp32", (544, 505, 427, 3), "separate"), ("fp32", (545, 505, 427, 3), "bricks"), ("fp32", (628, 303, 256, 3), "separate"),
+    ("fp32", (676, 303, 256, 3), "bricks"), ("fp32", (464, 464, 464, 1), "separate"), ("fp32", (464, 464, 400, 1), "bricks"),
+    ("fp32", (464, 464, 551, 1), "bricks"), ("fp32", (416, 464, 464, 1), "bricks"), ("fp32", (400, 400, 400, 4), "bricks"),
+    ("fp64", (353, 353, 353, 4), "separate"), ("fp64", (353, 353, 353, 2), "bricks"), ("fp64", (352, 353, 353, 4), "bricks"),
+    ("fp64", (354, 353, 353, 4), "bricks"), ("fp64", (353, 353, 385, 4), "bricks"), ("fp64", (514, 353, 353, 1), "bricks"),
+    ("fp64", (514, 353, 353, 3), "separate"), ("fp64", (400, 400, 400, 4), "bricks")])
+def test_bricks_only_where_they_pay(pkg, precision, shape, form):
+    assert planned(pkg, shape, precision)[0] == form
