@@ -18,10 +18,12 @@ sweep kernels on the GPU (HIP events around each launch, via
   advances together (``Microenvironment.set_col_runs``), per axis;
 * schedule: whole-volume sweeps, the two substrate halves swept on parallel
   streams, or (FP64) x/y sweeps in k-slabs of a few planes, the slabs with
-  each of the three fastest wave x chunk lengths (chosen by graph-replayed
-  whole-step time; slabs have to win by 2 %);
-* the library's default schedule, which may sweep x and y together: it is
-  kept, as shapes of 0, when its whole step is the fastest.
+  each of the three fastest wave x chunk lengths (chosen by whole-step time;
+  slabs have to win by 2 %);
+* the library's default schedule where it sweeps x and y together
+  (``Microenvironment.schedule``), with its best z tile runs and one or two
+  substrate streams: it is kept, as shapes of 0, when its whole step is the
+  fastest.
 
 Results are cached per (nx, ny, nz, ns, precision) in memory and, when a path
 is given, in a JSON file.
@@ -65,10 +67,10 @@ def _time(env, dt, reps, shape):
 
 
 def _step_ms(env, dt, reps):
-    """Mean graph-replayed step time (ms) over 2*reps + 2 steps."""
+    """Mean step time (ms) over 2*reps + 2 steps."""
     import time
 
-    env.step(dt, 2)  # capture the schedule's graph
+    env.step(dt, 2)  # tables of the fused sweep, the graph of a large field's step
     env.synchronize()
     n = 2 * reps + 2
     t0 = time.perf_counter()
@@ -96,6 +98,8 @@ def autotune(pkg, nx, ny, nz, ns, precision="fp32", dt=0.01, reps=6, cache_path=
     env = pkg.Microenvironment(nx, ny, nz, ns, 20.0, precision)
     trials = []
     try:
+        # whether the default schedule is one that the shapes searched below cannot reach
+        together = hasattr(env, "schedule") and env.schedule()[0] != "separate"
         env.set_coefficients(10 ** rng.uniform(3, 5, ns), rng.uniform(0.01, 1, ns))
         env.set_dirichlet(np.ones(ns, np.uint8), np.ones(6, np.uint8), np.full((6, ns), 20.0))
         if nx * ny * nz * ns <= 1 << 27:
@@ -163,7 +167,7 @@ def autotune(pkg, nx, ny, nz, ns, precision="fp32", dt=0.01, reps=6, cache_path=
             if ms[2] < best_rz[0]:
                 best_rz = (ms[2], R)
         env.set_col_runs(best_ry[1], best_rz[1])
-        # schedules, by graph-replayed step time: whole-volume sweeps, the two
+        # schedules, by step time: whole-volume sweeps, the two
         # substrate halves on parallel streams, x/y k-slabs.  The k-slab
         # schedule runs the x sweep of one slab beside the y sweep of the one
         # before, and the x chunk length that is fastest alone is not always
@@ -217,21 +221,27 @@ def autotune(pkg, nx, ny, nz, ns, precision="fp32", dt=0.01, reps=6, cache_path=
                "trials": trials}
         # the default schedule (400^3 x 4: 1.00 ms FP32 and 1.68 ms FP64 against
         # 1.22 and 2.18 with the best separate sweeps)
-        try:
+        if together:
             env.set_tiles(0, 0, 0, 0, 0, 0)
-            default = True
-        except Exception:
-            default = False
-        if default:
             env.set_x_grid(0)
-            env.set_col_runs(1, 1)
-            t = _step_ms(env, dt, reps)
-            trials.append({"axis": "schedule", "default": True, "ms_step": t})
-            if t < best_sched[0]:
+            best_rz = None
+            for R in COL_RUNS:
+                env.set_col_runs(1, R)
+                env.time_kernels(dt, 1)
                 ms = env.time_kernels(dt, reps)
-                res.update({"Lx": 0, "rows_x": 0, "Ly": 0, "cols_y": 0, "Lz": 0, "cols_z": 0, "x_grid": 0,
-                            "runs_y": 1, "runs_z": 1, "slab": 0, "substrate_streams": 1,
-                            "ms": {"x": ms[0], "y": ms[1], "z": ms[2], "step": t}})
+                trials.append({"axis": "z", "default": True, "runs": R, "ms_z": ms[2]})
+                if best_rz is None or ms[2] < best_rz[0][2]:
+                    best_rz = (ms, R)
+            env.set_col_runs(1, best_rz[1])
+            for split in (1, 2) if ns > 1 else (1,):
+                env.set_substrate_streams(split)
+                t = _step_ms(env, dt, reps)
+                trials.append({"axis": "schedule", "default": True, "slab": 0, "substrate_streams": split, "ms_step": t})
+                if t < res["ms"]["step"]:
+                    ms = best_rz[0]
+                    res.update({"Lx": 0, "rows_x": 0, "Ly": 0, "cols_y": 0, "Lz": 0, "cols_z": 0, "x_grid": 0,
+                                "runs_y": 1, "runs_z": best_rz[1], "slab": 0, "substrate_streams": split,
+                                "ms": {"x": ms[0], "y": ms[1], "z": ms[2], "step": t}})
     finally:
         env.close()
     if verbose:
@@ -256,7 +266,7 @@ def autotune_agents(env, dt=0.01, steps=20, reps=2):
     step stores the field (whole 128-byte lines or single voxels) and, with
     several substrates and no k-slab schedule, whether the two substrate
     halves run on parallel streams (each half's agent step then overlaps the
-    other half's sweeps), by graph-replayed step time; the fastest pair is
+    other half's sweeps), by step time; the fastest pair is
     left set.  Every trial advances the field (reps * (steps + 4) steps per
     candidate): tune before the run.  Returns {"whole_lines",
     "substrate_streams", "ms_step": {(whole_lines, streams): ms}}."""
