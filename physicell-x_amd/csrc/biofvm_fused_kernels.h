@@ -65,9 +65,8 @@ __device__ __forceinline__ double lane_get(double v, int from) {
 // tested for its place in the row: the Dirichlet ends are set in LDS first,
 // coefficients past the row end are zero (so the padding solves to zero), and
 // the first padded node repeats the last one, which makes the FP32 form's link
-// past the row end vanish.  Lanes without a row (on false) solve the values that
-// `row` points to and do not store; these have to be finite, since a scan step
-// that is off still multiplies another row's value by zero.
+// past the row end vanish.  Lanes without a row (on false) solve the row that
+// `row` points to and do not store.
 template <typename T, int L, bool DEV>
 __device__ __forceinline__ void lds_row_solve(T* __restrict__ row, bool on, int nx, int p, int P, bool dact, T v_lo,
                                               T v_hi, const T* __restrict__ s_xi, const T* __restrict__ s_xc,
@@ -222,10 +221,19 @@ __device__ __forceinline__ void sweep_xy_plane(const PlaneShape<T>& g, const Swe
     const int t = threadIdx.x, nthr = blockDim.x, lane = t & 63, nw = nthr >> 6;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     T* plane = a.u + (long long)d * a.N + (long long)k * ny * nx;
+    // Held rows on a y face start from zero: the Dirichlet passes set them below
+    // whatever they hold, and a NaN or infinity there would reach the rows that
+    // share the wavefront (a scan step that is off multiplies another row's value
+    // by zero).  Not loading them costs nothing; leaving them out of the x phase
+    // cost 1 to 5 % of this kernel (64^3 x 2 FP64 12.2 -> 12.9 us).
+    const bool dact = (a.active >> d) & 1ull;
+    const int jlo = dact ? 1 : 0, jhi = dact ? ny - 1 : ny;
     if (g.vec)
-        rows_to_lds<T, 16, 0>(tile, S, plane, nx, ny, wave, nw, lane);
+        rows_to_lds<T, 16, 0>(tile + jlo * S, S, plane + jlo * nx, nx, jhi - jlo, wave, nw, lane);
     else
-        rows_to_lds<T, 4, 0>(tile, S, plane, nx, ny, wave, nw, lane);
+        rows_to_lds<T, 4, 0>(tile + jlo * S, S, plane + jlo * nx, nx, jhi - jlo, wave, nw, lane);
+    if (dact)
+        for (int e = t; e < nx; e += nthr) tile[e] = tile[(ny - 1) * S + e] = T(0);
     for (int e = t; e < P * L; e += nthr) {
         s_xi[e] = e < nx ? a.inv[(long long)d * nx + e] : T(0);
         s_xc[e] = e < nx ? a.cp[(long long)d * nx + e] : T(0);
@@ -239,7 +247,6 @@ __device__ __forceinline__ void sweep_xy_plane(const PlaneShape<T>& g, const Swe
             tile[r * S + nx + e - r * pad] = T(0);
         }
     }
-    const bool dact = (a.active >> d) & 1ull;
     const T kd = a.k[d], lam = DEV ? a.k[a.ns + d] : T(0), bt = DEV ? a.beta[d] : T(0);
     const T v_lo = PV ? T(0) : a.dval[dir_slot_xonly(0, nx, a.reg) * a.ns + d];
     const T v_hi = PV ? T(0) : a.dval[dir_slot_xonly(nx - 1, nx, a.reg) * a.ns + d];
@@ -257,15 +264,11 @@ __device__ __forceinline__ void sweep_xy_plane(const PlaneShape<T>& g, const Swe
         }
         __syncthreads();
     }
-    // x phase.  Held rows on a y face are left out: the Dirichlet passes set them
-    // below whatever they hold, and a NaN or infinity there would reach the rows
-    // that share the wavefront.  Held planes are solved too and overwritten whole.
-    const int jlo = dact ? 1 : 0, jhi = dact ? ny - 1 : ny;
+    // x phase.  Rows on a y or z face are solved too and overwritten below.
     for (int r = wave * RW; r < ny; r += nw * RW) {
-        const int j = r + rw;
-        const bool on = rw < RW && j >= jlo && j < jhi;
-        lds_row_solve<T, L, DEV>(on ? tile + j * S : s_xi, on, nx, p, P, dact && !PV, v_lo, v_hi, s_xi, s_xc, s_sm, kd,
-                                 lam, bt);
+        const bool on = rw < RW && r + rw < ny;
+        lds_row_solve<T, L, DEV>(tile + (on ? r + rw : r) * S, on, nx, p, P, dact && !PV, v_lo, v_hi, s_xi, s_xc,
+                                 s_sm, kd, lam, bt);
     }
     __syncthreads();
     // y phase: thread (yi, py) owns rows [py*LY, py*LY + LY) of column c0 + yi
@@ -611,10 +614,17 @@ __global__ __launch_bounds__(1024) void k_sweep_xy_brick(BrickArgs<T> g) {
     const int hl = DEV && j0 > 0 ? 1 : 0, hr = DEV && j1 < ny ? 1 : 0;
     const int nrx = nr + hl + hr;
     const T* src = a.u + (long long)d * a.N + (long long)(k * ny + j0 - hl) * nx;
+    // held rows start from zero as in sweep_xy_plane
+    const bool dact = (a.active >> d) & 1ull;
+    const int rlo = dact && j0 == 0 ? 1 : 0, rhi = dact && j1 == ny ? nrx - 1 : nrx;
     if (g.vec)
-        rows_to_lds<T, 16, kStream>(tile, S, src, nx, nrx, wave, nw, lane);
+        rows_to_lds<T, 16, kStream>(tile + rlo * S, S, src + rlo * nx, nx, rhi - rlo, wave, nw, lane);
     else
-        rows_to_lds<T, 4, kStream>(tile, S, src, nx, nrx, wave, nw, lane);
+        rows_to_lds<T, 4, kStream>(tile + rlo * S, S, src + rlo * nx, nx, rhi - rlo, wave, nw, lane);
+    if (rlo > 0)
+        for (int e = t; e < nx; e += nthr) tile[e] = T(0);
+    if (rhi < nrx)
+        for (int e = t; e < nx; e += nthr) tile[rhi * S + e] = T(0);
     for (int e = t; e < P * L; e += nthr) {
         s_xi[e] = e < nx ? a.inv[(long long)d * nx + e] : T(0);
         s_xc[e] = e < nx ? a.cp[(long long)d * nx + e] : T(0);
@@ -629,7 +639,6 @@ __global__ __launch_bounds__(1024) void k_sweep_xy_brick(BrickArgs<T> g) {
     }
     // rows past the brick (their y coefficients are zero)
     for (int e = nrx * S + t; e < kRows * S; e += nthr) tile[e] = T(0);
-    const bool dact = (a.active >> d) & 1ull;
     const T kd = a.k[d], lam = DEV ? a.k[a.ns + d] : T(0), bt = DEV ? a.beta[d] : T(0);
     const T v_lo = a.dval[dir_slot_xonly(0, nx, a.reg) * a.ns + d];
     const T v_hi = a.dval[dir_slot_xonly(nx - 1, nx, a.reg) * a.ns + d];
@@ -640,11 +649,10 @@ __global__ __launch_bounds__(1024) void k_sweep_xy_brick(BrickArgs<T> g) {
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's rows are in LDS
     __syncthreads();
-    // x phase: RW rows per wavefront, held rows left out as in sweep_xy_plane
-    const int rlo = dact && j0 == 0 ? 1 : 0, rhi = dact && j1 == ny ? nrx - 1 : nrx;
+    // x phase: RW rows per wavefront
     for (int r = wave * RW; r < nrx; r += nw * RW) {
-        const bool on = rw < RW && r + rw >= rlo && r + rw < rhi;
-        lds_row_solve<T, L, DEV>(on ? tile + (r + rw) * S : s_xi, on, nx, p, P, dact, v_lo, v_hi, s_xi, s_xc, s_sm, kd, lam,
+        const bool on = rw < RW && r + rw < nrx;
+        lds_row_solve<T, L, DEV>(tile + (on ? r + rw : r) * S, on, nx, p, P, dact, v_lo, v_hi, s_xi, s_xc, s_sm, kd, lam,
                                  bt);
     }
     __syncthreads();
