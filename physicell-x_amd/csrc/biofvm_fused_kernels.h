@@ -8,8 +8,10 @@
 //    one launch takes the place of three (x sweep, face pass, y sweep).
 //  * Fields larger than the last-level cache (k_sweep_xy_brick): a block per
 //    brick of consecutive rows.  Three separate sweeps move such a field six
-//    times; with y lines cut at the brick borders it moves four times.  With
-//    T_c the rows of brick c of the line's matrix and k = D*dt/dx^2 the
+//    times; with y lines cut at the brick borders it moves four times.  (The
+//    cut is that of the SPIKE method of Polizzi and Sameh, Parallel Computing
+//    32, 2006: block diagonal solves, a reduced system of the border values,
+//    and spikes that carry them back.)  With T_c the rows of brick c of the line's matrix and k = D*dt/dx^2 the
 //    coupling across a border,
 //      x_c = T_c^-1 r_c + SL_c * E_(c-1) + SR_c * F_(c+1),
 //      SL_c = k T_c^-1 e_first,  SR_c = k T_c^-1 e_last,
@@ -163,12 +165,14 @@ __global__ __launch_bounds__(64) void k_scan_multipliers(int nx, int L, const T*
 // dealt to the wavefronts.  Complete after this thread's s_waitcnt vmcnt(0)
 // and a barrier.  16 bytes per lane need rows of whole 16-byte vectors (a
 // longer load would write into the padding).  AUX: cache policy of the loads
-// (kStream where the field is larger than the caches).
+// (kStream where the field is larger than the caches).  Returns the wavefront's
+// last row (negative if it has none).
 constexpr int kStream = 2;
 template <typename T, int B, int AUX>
-__device__ __forceinline__ void rows_to_lds(T* tile, int S, const T* src, int nx, int rows, int wave, int nw, int lane) {
+__device__ __forceinline__ int rows_to_lds(T* tile, int S, const T* src, int nx, int rows, int wave, int nw, int lane) {
     const int bytes = nx * (int)sizeof(T);
-    for (int r = wave; r < rows; r += nw) {
+    int r = wave;
+    for (; r < rows; r += nw) {
         const char* g = reinterpret_cast<const char*>(src + (long long)r * nx);
         char* l = reinterpret_cast<char*>(tile + r * S);
         for (int o = 0; o < bytes; o += 64 * B)
@@ -181,6 +185,7 @@ __device__ __forceinline__ void rows_to_lds(T* tile, int S, const T* src, int nx
                     __builtin_amdgcn_global_load_lds(from, to, 4, 0, AUX);
             }
     }
+    return r - nw;
 }
 
 // ---- one plane per block -----------------------------------------------------------
@@ -589,7 +594,7 @@ __global__ __launch_bounds__(64) void k_chunk_products(int n, int L, const T* __
 // values, needs no halo and works in place.
 // Bound by HBM with the x phase of one block under the loads of the other (two
 // 512-thread blocks per CU).  400^3 x 4: 830 us FP64 (4.9 TB/s; x and y sweep:
-// 1700), 490 us FP32 (4.2 TB/s; 870).
+// 1700), 465 us FP32 (4.4 TB/s; 870).
 // Dynamic LDS, of T: (LY, FP32 LY + 2)*S tile | 2*roundup4(LY) y coefficients |
 // 2*P*L x coefficients | 12*P scan multipliers.
 template <typename T, int L, int LY, bool DEV>
@@ -614,17 +619,8 @@ __global__ __launch_bounds__(1024) void k_sweep_xy_brick(BrickArgs<T> g) {
     const int hl = DEV && j0 > 0 ? 1 : 0, hr = DEV && j1 < ny ? 1 : 0;
     const int nrx = nr + hl + hr;
     const T* src = a.u + (long long)d * a.N + (long long)(k * ny + j0 - hl) * nx;
-    // held rows start from zero as in sweep_xy_plane
-    const bool dact = (a.active >> d) & 1ull;
-    const int rlo = dact && j0 == 0 ? 1 : 0, rhi = dact && j1 == ny ? nrx - 1 : nrx;
-    if (g.vec)
-        rows_to_lds<T, 16, kStream>(tile + rlo * S, S, src + rlo * nx, nx, rhi - rlo, wave, nw, lane);
-    else
-        rows_to_lds<T, 4, kStream>(tile + rlo * S, S, src + rlo * nx, nx, rhi - rlo, wave, nw, lane);
-    if (rlo > 0)
-        for (int e = t; e < nx; e += nthr) tile[e] = T(0);
-    if (rhi < nrx)
-        for (int e = t; e < nx; e += nthr) tile[rhi * S + e] = T(0);
+    const int last = g.vec ? rows_to_lds<T, 16, kStream>(tile, S, src, nx, nrx, wave, nw, lane)
+                           : rows_to_lds<T, 4, kStream>(tile, S, src, nx, nrx, wave, nw, lane);
     for (int e = t; e < P * L; e += nthr) {
         s_xi[e] = e < nx ? a.inv[(long long)d * nx + e] : T(0);
         s_xc[e] = e < nx ? a.cp[(long long)d * nx + e] : T(0);
@@ -639,6 +635,7 @@ __global__ __launch_bounds__(1024) void k_sweep_xy_brick(BrickArgs<T> g) {
     }
     // rows past the brick (their y coefficients are zero)
     for (int e = nrx * S + t; e < kRows * S; e += nthr) tile[e] = T(0);
+    const bool dact = (a.active >> d) & 1ull;
     const T kd = a.k[d], lam = DEV ? a.k[a.ns + d] : T(0), bt = DEV ? a.beta[d] : T(0);
     const T v_lo = a.dval[dir_slot_xonly(0, nx, a.reg) * a.ns + d];
     const T v_hi = a.dval[dir_slot_xonly(nx - 1, nx, a.reg) * a.ns + d];
@@ -648,6 +645,12 @@ __global__ __launch_bounds__(1024) void k_sweep_xy_brick(BrickArgs<T> g) {
         s_cp[t] = g.ycp[((long long)d * C + cb) * LY + t];
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's rows are in LDS
+    // held rows are cleared, as in sweep_xy_plane, by the wavefront that loaded
+    // them (not loading them took 950 us where this takes 929, 400^3 x 4 FP64)
+    if (dact && j0 == 0 && wave == 0)
+        for (int e = lane; e < nx; e += 64) tile[e] = T(0);
+    if (dact && j1 == ny && last == nrx - 1)
+        for (int e = lane; e < nx; e += 64) tile[last * S + e] = T(0);
     __syncthreads();
     // x phase: RW rows per wavefront
     for (int r = wave * RW; r < nrx; r += nw * RW) {
