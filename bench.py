@@ -81,11 +81,14 @@ def make_workload(n, ns, n_agents, seed):
                 S=S, U=U, E=E, rs=rs, V=V)
 
 
-def swept_together(slab, ms):
-    """Whether the x slot of the kernel times holds the x and the y sweep: the
-    k-slab schedule, or one kernel for both (the y slot is then an empty event
-    pair)."""
-    return slab > 0 or ms[1] < 0.05 * ms[0]
+def sweep_names(schedule, slab):
+    """Names of the kernels behind the x, y and z slots of the kernel times, from
+    Microenvironment.schedule(): "xy_slab" for the k-slab schedule, "xy" for one
+    kernel that sweeps both (with bricks also the border solve; the y slot is
+    then an empty event pair), and "z_fix" for the z sweep of a bricked field."""
+    if slab:
+        return ["xy_slab", "y", "z"]
+    return {"separate": ["x", "y", "z"], "planes": ["xy", "y", "z"], "bricks": ["xy", "y", "z_fix"]}[schedule[0]]
 
 
 def make_env(pkg, w, n, ns, precision, tiles=None, tune_agents=False):
@@ -160,12 +163,14 @@ def run_host_boundary(env, dt, updates, prec, reps=3, fix_basis=False):
             "pcie_bytes_down": int(host.size * (4 if fp32 else 8)), "reps": reps}
 
 
-def load_traffic(kernel_key, tiles):
+def load_traffic(kernel_key, tiles, schedule=("separate",)):
     """(HBM bytes per launch, y and z tile sub-runs of the counter run) of a
     sweep kernel, from the counter runs recorded in profiles/traffic.json, or
     (None, None) unless an entry was measured with this exact kernel shape
     (tiles = Lx, Ly, Lz, rows_x, cols_y, cols_z): another shape moves other
-    bytes, so its figure is not reported.  The tile order (sub-runs per XCD)
+    bytes, so its figure is not reported; kernels that sweep x and y together
+    and the z sweep after them are matched by their schedule instead
+    (Microenvironment.schedule()).  The tile order (sub-runs per XCD)
     only changes which block solves which tile, and the counters read the
     same bytes for every order measured (z at 400^3 and 800^3: 1.000x at one
     run and at the tuned count), so an entry of another order is reported,
@@ -177,7 +182,8 @@ def load_traffic(kernel_key, tiles):
         ent = json.load(open(path)).get("entries", {}).get(kernel_key)
     except Exception:
         return None, None
-    if not ent or [int(t) for t in ent.get("tiles", [])] != [int(t) for t in list(tiles)[:6]]:
+    shape = [int(t) for t in list(tiles)[:6]] if schedule[0] == "separate" else list(schedule)
+    if not ent or ent.get("tiles" if schedule[0] == "separate" else "schedule") != shape:
         return None, None
     return ent.get("bytes"), [int(r) for r in ent.get("runs", [1, 1])]
 
@@ -554,13 +560,12 @@ def run_large(pkg, n=800, steps=20, seed=3, tune=True, fixed=None):
         dt_ = time.perf_counter() - t0
         ms = e.time_kernels(0.01, 5)
         tsize = 4 if prec == "fp32" else 8
-        joint = swept_together(e.slab(), ms)
-        names = ["xy_slab" if e.slab() else "xy" if joint else "x", "y", "z"]
+        names = sweep_names(e.schedule(), e.slab())
         dom = int(np.argmax(ms[:3]))
         sweeps = 2 if (e.slab() and dom == 0) else 1  # passes over the field (one kernel for both: one)
         alg = updates * 2 * tsize * sweeps
         achieved = alg / (ms[dom] * 1e-3) / 1e9
-        traf = load_traffic(f"sweep_{names[dom]}_{prec}_{n}", e.tiles())
+        traf = load_traffic(f"sweep_{names[dom]}_{prec}_{n}", e.tiles(), e.schedule())
         out[prec] = {"value": updates * (steps - 1) / dt_, "ms_per_step": 1e3 * dt_ / (steps - 1),
                      "step_alg_frac_of_peak": updates * 6 * tsize / (dt_ / (steps - 1)) / 1e9 / PEAK_HBM_GBS,
                      "kernel_ms": dict(x=ms[0], y=ms[1], z=ms[2], agents=ms[3]),
@@ -570,7 +575,7 @@ def run_large(pkg, n=800, steps=20, seed=3, tune=True, fixed=None):
                                   "frac": achieved / PEAK_HBM_GBS,
                                   "traffic": traf[0], "traffic_col_runs": traf[1]},
                      "tiles": list(e.tiles()), "autotuned": tune and (fixed or {}).get(prec) is None,
-                     "schedule": {"slab": e.slab(), "substrate_streams": e.substrate_streams(),
+                     "schedule": {"xy": list(e.schedule()), "slab": e.slab(), "substrate_streams": e.substrate_streams(),
                                   "x_grid": e.x_grid()[0], "runs_y": e.col_runs()[0], "runs_z": e.col_runs()[1]},
                      "agent_stores": "whole lines" if e.agent_stores() else "single voxels"}
         envs[prec] = e
@@ -654,6 +659,7 @@ def main():
     env32 = make_env(pkg, w, n, ns, "fp32", tiles["fp32"], tune_agents=tune_ag and not args.tiles)
     wall32, ms32, gwall32 = time_gpu(env32, dt, args.steps, args.warmup)
     tiles32 = env32.tiles()
+    sched32 = env32.schedule()
     runs32 = env32.col_runs()
     lines32 = env32.agent_stores()
     split32 = env32.substrate_streams()
@@ -670,7 +676,7 @@ def main():
         res["fp64"] = dict(value=updates * args.steps / wall64, ms_per_step=1e3 * wall64 / args.steps,
                            eager_ms_per_step=1e3 * gwall64 / args.steps,
                            kernel_ms=dict(x=ms64[0], y=ms64[1], z=ms64[2], agents=ms64[3]),
-                           tiles=list(env64.tiles()), col_runs=list(env64.col_runs()),
+                           tiles=list(env64.tiles()), xy=list(env64.schedule()), col_runs=list(env64.col_runs()),
                            substrate_streams=env64.substrate_streams(), slab=env64.slab(),
                            agent_stores="whole lines" if env64.agent_stores() else "single voxels")
         res["fp32_vs_fp64"] = dict(max_rel_err_per_substrate=errs, mass_drift_per_substrate=drift,
@@ -686,12 +692,12 @@ def main():
     env32.close()
 
     slab32 = tiles["fp32"]["slab"] if tiles["fp32"] else 0
-    names = ["xy_slab" if slab32 else "xy" if swept_together(slab32, ms32) else "x", "y", "z"]
+    names = sweep_names(sched32, slab32)
     dom = int(np.argmax(ms32[:3]))
     sweeps = 2 if (slab32 and dom == 0) else 1
     alg_bytes = updates * 2 * 4 * sweeps  # one FP32 read + one write per voxel-substrate per sweep
     achieved = alg_bytes / (ms32[dom] * 1e-3) / 1e9
-    traffic, traffic_runs = load_traffic(f"sweep_{names[dom]}_fp32_{n}", tiles32)
+    traffic, traffic_runs = load_traffic(f"sweep_{names[dom]}_fp32_{n}", tiles32, sched32)
     out = {
         "metric": METRIC,
         "value": updates * args.steps / wall32,
@@ -718,7 +724,7 @@ def main():
         "copy_stream_GBps": copy_stream_gbs,
         "eager_ms_per_step": 1e3 * gwall32 / args.steps,
         "tiles": dict(Lx=tiles32[0], Ly=tiles32[1], Lz=tiles32[2], rows_x=tiles32[3],
-                      cols_y=tiles32[4], cols_z=tiles32[5], slab=slab32,
+                      cols_y=tiles32[4], cols_z=tiles32[5], xy=list(sched32), slab=slab32,
                       substrate_streams=split32,
                       x_grid=(tiles["fp32"] or {}).get("x_grid", 0),
                       runs_y=runs32[0], runs_z=runs32[1],

@@ -306,8 +306,9 @@ int bfa_get_substrate_streams(const bfa_env *env);
  * unit (capped at how many fit), each wavefront striding over row groups; 0
  * (the default) launches as many as fit.  Fewer resident waves can stream
  * faster (at 400^3 x 4 FP32, 4 blocks per CU instead of the 5 that fit);
- * the autotuner measures it.  bfa_get_x_grid reports the requested value
- * and how many fit for the current shape.  No reference counterpart (a
+ * the autotuner measures it.  Without effect where x and y are swept together
+ * (bfa_get_schedule).  bfa_get_x_grid reports the requested value and how many
+ * fit for the current shape.  No reference counterpart (a
  * launch parameter of the x sweep, BioFVM/BioFVM_solvers.cpp:352-426). */
 int bfa_set_x_grid(bfa_env *env, int blocks_per_cu);
 int bfa_get_x_grid(const bfa_env *env, int *requested, int *resident);
@@ -317,8 +318,8 @@ int bfa_get_x_grid(const bfa_env *env, int *requested, int *resident);
  * (runs_z) sub-runs that it advances together, so that the blocks it holds at
  * one time read from that many separate stretches of the field; 1 (the
  * default) is one contiguous run.  The arithmetic per line is the same, so
- * results are bit-identical for every value.  Range [1, 64]; the autotuner
- * measures it (at 400^3 x 4 FP32 the z sweep is fastest with a few runs).
+ * results are bit-identical for every value; runs_y is without effect where x
+ * and y are swept together.  Range [1, 64]; the autotuner measures it (at 400^3 x 4 FP32 the z sweep is fastest with a few runs).
  * No reference counterpart (a launch parameter of the y and z sweeps,
  * BioFVM/BioFVM_solvers.cpp:427-777). */
 int bfa_set_col_runs(bfa_env *env, int runs_y, int runs_z);

@@ -931,11 +931,14 @@ int enqueue_step(bfa_env* e) {
 // several steps replay as fast as kernels but take 0.6 to 1.7 ms to build.  The
 // slab and substrate schedules have tens of launches and events per step, which
 // a graph replays faster than the host can enqueue them.  Fields above 40 MiB
-// keep the graph too: their steps take 60 us and more, and hundreds of kernels
-// enqueued ahead made a program with busy host threads unsteady (203x157x121 x
-// 3 FP32, 100 steps and a save in single precision: 9.7 to 9.9 ms as graphs,
-// 10.3 to 11.9 as kernels over eleven runs; 131x257x67 x 2 FP64, 34 MiB: 7.6 as
-// graphs, 7.2 as kernels).
+// keep the graph too: their steps take 60 us and more, kernels gain nothing
+// there, and hundreds of kernels enqueued ahead made a program with busy host
+// threads unsteady (203x157x121 x 3 FP32, 44 MiB, 100 steps and a save in single
+// precision: 9.7 to 9.9 ms as graphs, 10.3 to 11.9 as kernels over eleven runs).
+// 100 steps and a save, graphs and kernels, medians of 15: FP32 128^3 x 2 5.2 /
+// 4.4 ms, 170x160x150 x 2 (31 MiB) 7.6 / 7.1, 210^3 (35) 9.3 / 8.9, 180x240x230
+// (38) 9.2 / 8.8, 250x250x200 (48) 9.4 / 9.5; FP64 150^3 (26) 5.7 / 5.3,
+// 131x257x67 x 2 (34) 7.3 / 6.9, 180x170x180 (42) 7.7 / 7.7.
 bool step_as_graph(const bfa_env* e) {
     if ((size_t)e->N * e->ns * e->tsize > (size_t)40 << 20) return true;
     return e->hplanes.empty() && ((e->slab > 0 && e->R == 0) || split_schedule(e));

@@ -11,8 +11,8 @@
 //    times; with y lines cut at the brick borders it moves four times.  (The
 //    cut is that of the SPIKE method of Polizzi and Sameh, Parallel Computing
 //    32, 2006: block diagonal solves, a reduced system of the border values,
-//    and spikes that carry them back.)  With T_c the rows of brick c of the line's matrix and k = D*dt/dx^2 the
-//    coupling across a border,
+//    and spikes that carry them back.)  With T_c the rows of brick c of the
+//    line's matrix and k = D*dt/dx^2 the coupling across a border,
 //      x_c = T_c^-1 r_c + SL_c * E_(c-1) + SR_c * F_(c+1),
 //      SL_c = k T_c^-1 e_first,  SR_c = k T_c^-1 e_last,
 //    where F and E are the line's values at a brick's first and last row.  The

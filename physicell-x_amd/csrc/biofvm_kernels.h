@@ -59,9 +59,10 @@ struct SweepArgs {
     const T* beta;    // [ns] deviation shift (FP32 form), unused for FP64
     const T* dval;    // [7][ns] Dirichlet value per face slot
     // Per-voxel Dirichlet values of the six face planes, or nullptr to use
-    // dval; read only by the standalone face pass (k_dirichlet_faces): with
-    // planes the sweeps apply no Dirichlet values themselves and the face
-    // pass runs between them.  Substrate d's planes start at plane + d*shell,
+    // dval.  The separate sweeps then apply no Dirichlet values and the face
+    // pass (k_dirichlet_faces) runs between them; the plane kernel
+    // (sweep_xy_plane) applies the first three passes itself, and the face pass
+    // after the z sweep is left.  Substrate d's planes start at plane + d*shell,
     // in the order
     //   xmin [k][j], xmax [k][j]   (ny*nz each)
     //   ymin [k][i], ymax [k][i]   (nx*nz each)
