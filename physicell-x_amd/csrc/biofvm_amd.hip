@@ -384,10 +384,11 @@ int choose_tiles(bfa_env* e) {
     return BFA_OK;
 }
 
-// Dynamic LDS up to the device's limit for a kernel.  The limit belongs to the
-// kernel, which every environment shares: set to one environment's need, it
-// would fall below what another one launches with.
-bool allow_lds(const bfa_env* e, const void* fn) {
+// Lets a kernel launch with `need` bytes of dynamic LDS.  The limit belongs to
+// the kernel, which every environment shares: set to one environment's need, it
+// would fall below what another one launches with, so it is the device's.
+bool allow_lds(const bfa_env* e, const void* fn, size_t need) {
+    if (need <= 65536) return true;  // any kernel's
     if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, e->max_lds) == hipSuccess) return true;
     (void)hipGetLastError();
     return false;
@@ -558,7 +559,7 @@ int raise_lds_limits(bfa_env* e) {
                             lds_col(e, e->nz, e->L[2], e->TX[2])};
     const void* fn[3] = {fx, fy, fz};
     for (int a = 0; a < 3; ++a)
-        if (need[a] > 65536 && fn[a] && !allow_lds(e, fn[a]))
+        if (fn[a] && !allow_lds(e, fn[a], need[a]))
             return fail(e, BFA_ERR_HIP, "axis %d: %zu bytes of LDS refused", a, need[a]);
     if (e->R == 0) {
         const void* fw = nullptr;
@@ -641,12 +642,12 @@ void invalidate_graph(bfa_env* e);
 
 #include "biofvm_fused_host.inc"
 
-// Kept agent blocks, and the memory of the fused sweep: the handle runs the
-// separate sweeps from then on.
+// Kept agent blocks, and the memory of bricks: the handle runs the separate
+// sweeps from then on.
 bool reclaim(bfa_env* e) {
-    const bool any = !e->spare.empty() || e->xy.sm;
+    const bool bricks = e->xy.C > 0 && e->xy.sm, any = !e->spare.empty() || bricks;
     free_spare(e);
-    if (e->xy.sm) {
+    if (bricks) {
         invalidate_graph(e);
         (void)hipStreamSynchronize(e->stream);
         free_fused(e);
@@ -1260,7 +1261,7 @@ int bfa_set_dirichlet_planes(bfa_env* e, const double* planes) {
     e->shell = shell;
     e->hplanes.swap(h);
     e->pre_valid = false;
-    drop_unused_fused(e);
+    drop_unused_bricks(e);
     return BFA_OK;
 }
 
@@ -2126,7 +2127,7 @@ int bfa_set_tiles(bfa_env* e, int Lx, int Ly, int Lz, int rows_x, int cols_y, in
     }
     if (e->R != 0) e->slab = 0;
     invalidate_graph(e);
-    drop_unused_fused(e);
+    drop_unused_bricks(e);
     return BFA_OK;
 }
 
