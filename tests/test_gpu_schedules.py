@@ -223,3 +223,30 @@ def test_fp64_bricks_with_free_faces_and_windows(pkg, shape, rows, threads, diri
     ("fp64", (514, 353, 353, 3), "separate"), ("fp64", (400, 400, 400, 4), "bricks")])
 def test_bricks_only_where_they_pay(pkg, precision, shape, form):
     assert planned(pkg, shape, precision)[0] == form
+
+
+def test_memory_of_bricks_is_given_up_before_an_allocation_fails(pkg):
+    """800^3 x 20 FP64: the gradients of the field (246 GB) do not fit beside it
+    (82 GB).  The call fails as it did, and the handle has given its bricks up
+    (8 GB) first; it goes on with the separate sweeps."""
+    n, ns = 800, 20
+    room, card = ctypes.c_size_t(), ctypes.c_size_t()
+    L = pkg.lib()
+    assert L.hipMemGetInfo(ctypes.byref(room), ctypes.byref(card)) == 0
+    if room.value < 1.2e11 or card.value > 3.2e11:
+        pytest.skip("sized for a card of 288 GiB")
+    e = pkg.Microenvironment(n, n, n, ns, 20.0, "fp64")
+    try:
+        # zero decay and free faces: a uniform field stays as it is
+        e.set_coefficients(np.linspace(1e3, 1e5, ns), np.zeros(ns))
+        e.fill(np.arange(1.0, ns + 1))
+        e.step(0.01, 1)
+        assert e.schedule()[0] == "bricks"
+        before = e.total_mass()
+        one = np.zeros(1)
+        assert L.bfa_gradients(e._h, one.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), 1) == 4  # no memory
+        assert e.schedule() == ("separate",)
+        e.step(0.01, 1)
+        np.testing.assert_allclose(e.total_mass(), before, rtol=1e-12)
+    finally:
+        e.close()
