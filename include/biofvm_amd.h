@@ -276,7 +276,7 @@ int bfa_get_tiles(const bfa_env *env, int *out6);
  * columns per pass or bricks per plane, threads per block, dynamic LDS in
  * bytes}, form 0: separate sweeps (the rest 0), 1: whole k-planes, 2: bricks of
  * rows.  Bricks may still turn into separate sweeps in the first step, for want
- * of device memory. */
+ * of device memory or where D*dt/dx^2 exceeds 1024. */
 int bfa_get_schedule(const bfa_env *env, int *out6);
 
 /* Sweep schedule.  planes == 0: each sweep covers the whole volume.
@@ -319,7 +319,8 @@ int bfa_get_x_grid(const bfa_env *env, int *requested, int *resident);
  * one time read from that many separate stretches of the field; 1 (the
  * default) is one contiguous run.  The arithmetic per line is the same, so
  * results are bit-identical for every value; runs_y is without effect where x
- * and y are swept together.  Range [1, 64]; the autotuner measures it (at 400^3 x 4 FP32 the z sweep is fastest with a few runs).
+ * and y are swept together.  Range [1, 64]; the autotuner measures it (at
+ * 400^3 x 4 FP32 the separate z sweep is fastest with a few runs).
  * No reference counterpart (a launch parameter of the y and z sweeps,
  * BioFVM/BioFVM_solvers.cpp:427-777). */
 int bfa_set_col_runs(bfa_env *env, int runs_y, int runs_z);

@@ -50,6 +50,7 @@ constexpr size_t kFieldSlack = 64;
 struct FusedPlan {
     bool on = false;
     bool ready = false;  // the tables hold the current coefficients
+    bool stiff = false;  // D*dt/dx^2 is too large for bricks (note_stiffness)
     int L = 0, LY = 0, PY = 0, W = 0, threads = 0;  // kernel shape (PlaneArgs)
     size_t lds = 0;
     int C = 0;           // bricks per plane (0: whole planes)
@@ -852,6 +853,8 @@ int ensure_precompute(bfa_env* e, double dt) {
         return e->prec == BFA_FP32 ? fused_precompute<float>(e, e->pre_dt) : fused_precompute<double>(e, e->pre_dt);
     }
     invalidate_graph(e);
+    note_stiffness(e, dt);
+    drop_unused_bricks(e);
     int rc = e->prec == BFA_FP32 ? run_precompute<float>(e, dt) : run_precompute<double>(e, dt);
     if (rc) return rc;
     e->pre_dt = dt;

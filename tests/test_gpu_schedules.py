@@ -225,6 +225,35 @@ def test_bricks_only_where_they_pay(pkg, precision, shape, form):
     assert planned(pkg, shape, precision)[0] == form
 
 
+@pytest.mark.parametrize("shape,precision", [((180, 171, 60, 1), "fp32"), ((150, 130, 450, 4), "fp64")])
+def test_bricks_keep_the_bars_up_to_their_largest_k(pkg, shape, precision):
+    """k = D*dt/dx^2 up to 1000 against the oracle; from there on the separate
+    sweeps, bit for bit, and bricks again for a smaller dt."""
+    p = make_problem(*shape, seed=81, dirichlet="off")
+    p.decay[:] = 0.1
+    p.D[:] = 1000.0 * p.dx ** 2 / p.dt
+    e, sep = gpu_env(pkg, p, precision), gpu_env(pkg, p, precision)
+    try:
+        sep.set_tiles(*sep.tiles()[:3])
+        u = p.u0.copy()
+        oracle_for(p).diffusion_step(u, p.dt)
+        e.simulate_diffusion_decay(p.dt)
+        assert e.schedule()[0] == "bricks"
+        assert relmax(e.download(), u) <= TOL[precision]
+        for x in (e, sep):
+            x.upload(p.u0)
+            x.step(100 * p.dt, 2)
+        assert e.schedule() == ("separate",)
+        assert np.array_equal(e.download(), sep.download())
+        e.upload(p.u0)
+        e.step(p.dt, 1)
+        assert e.schedule()[0] == "bricks"
+        assert relmax(e.download(), u) <= TOL[precision]
+    finally:
+        e.close()
+        sep.close()
+
+
 def test_memory_of_bricks_is_given_up_before_an_allocation_fails(pkg):
     """800^3 x 20 FP64: the gradients of the field (246 GB) do not fit beside it
     (82 GB).  The call fails as it did, and the handle has given its bricks up
